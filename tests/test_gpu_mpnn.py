@@ -137,3 +137,22 @@ def test_trained_surrogate_saves_newton_iterations():
     assert max(h.residual_norm for h in fam.batch.histories) <= 1e-10
     assert diff <= 1e-9
     assert sum(itg) < sum(it0)
+
+
+def test_workspace_keeps_its_size_over_smaller_calls():
+    """a network first asked for many samples, then for a smaller minibatch (host features)
+    and again for many: the later calls' rows fit the workspace, and every answer is that
+    of a network that has seen nothing else"""
+    print("case mpnn workspace sizes", flush=True)
+    net, graph, X, T = _setup(n=17, nsamples=24, seed=5)
+    F = np.random.default_rng(6).normal(size=(24, X.shape[1]))
+    V = np.random.default_rng(7).uniform(-1, 1, (24, 4))
+    big = net.predict_sides(F, V)
+    loss, grad = net.loss_grad(X[:2], T[:2])
+    few = net.predict(X[:1])
+    again = net.predict_sides(F[:20], V[:20])
+    assert np.array_equal(again, big[:20])
+    assert np.isfinite(loss) and np.isfinite(grad).all()
+    net.train(X[:9], T[:9], epochs=1, batch=8)
+    fresh, _, _, _ = _setup(n=17, nsamples=1, seed=5)
+    assert np.array_equal(few, fresh.predict(X[:1]))

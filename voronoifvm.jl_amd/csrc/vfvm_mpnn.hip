@@ -689,6 +689,15 @@ void ensure_cap(vfvm_mpnn &m, int64_t rows) {
   m.cap = rows;
 }
 
+// host values into a workspace buffer of at least `count` entries (ensure_cap): the buffer
+// keeps its capacity, which later calls with more rows rely on.  Synchronous, as
+// DevBuf::upload.
+template <class T>
+void copy_in(DevBuf<T> &buf, const T *h, size_t count, hipStream_t st) {
+  VFVM_HIP_CHECK(hipMemcpyAsync(buf.p, h, count * sizeof(T), hipMemcpyHostToDevice, st));
+  VFVM_HIP_CHECK(hipStreamSynchronize(st));
+}
+
 // network input of `ns` samples: x16 = [x (8 features), smoothed context (8 channels)]
 void expand(vfvm_mpnn &m, const float *x, float *x16, int64_t ns) {
   hipStream_t st = m.ctx->stream;
@@ -1001,7 +1010,7 @@ int vfvm_mpnn_infer(vfvm_mpnn *m, int64_t nsamples, const float *features, doubl
     for (int64_t s0 = 0; s0 < nsamples; s0 += chunk) {
       const int64_t ns = std::min(chunk, nsamples - s0), rows = ns * m->n;
       ensure_cap(*m, rows);
-      m->x.upload(features + s0 * m->n * NFEAT, (size_t)rows * NFEAT, st);
+      copy_in(m->x, features + s0 * m->n * NFEAT, (size_t)rows * NFEAT, st);
       expand(*m, m->x.p, m->x16.p, ns);
       forward_infer(*m, rows);
       u.resize((size_t)rows);
@@ -1065,8 +1074,8 @@ int vfvm_mpnn_loss_grad(vfvm_mpnn *m, int64_t nsamples, const float *features, c
     hipStream_t st = m->ctx->stream;
     const int64_t rows = nsamples * m->n;
     ensure_cap(*m, rows);
-    m->x.upload(features, (size_t)rows * NFEAT, st);
-    m->target.upload(targets, (size_t)rows, st);
+    copy_in(m->x, features, (size_t)rows * NFEAT, st);
+    copy_in(m->target, targets, (size_t)rows, st);
     expand(*m, m->x.p, m->x16.p, nsamples);
     forward(*m, rows);
     const float lv = backward(*m, rows);
