@@ -156,3 +156,19 @@ def test_workspace_keeps_its_size_over_smaller_calls():
     net.train(X[:9], T[:9], epochs=1, batch=8)
     fresh, _, _, _ = _setup(n=17, nsamples=1, seed=5)
     assert np.array_equal(few, fresh.predict(X[:1]))
+
+
+@pytest.mark.parametrize("n,nsamples", [(6, 1), (17, 129), (41, 2), (150, 1), (203, 1)])
+def test_forward_matches_oracle_context_forms(n, nsamples):
+    """the context smoothing in LDS (one feature per block; both features, from 129 samples on;
+    more than 20480 nodes) and one launch per step (203 x 203 nodes do not fit the LDS)"""
+    print("case mpnn context", n, nsamples, flush=True)
+    net, graph, X, T = _setup(n=n, nsamples=nsamples, seed=n)
+    keep = [0, nsamples - 1]
+    u_gpu = net.predict(X)[keep]
+    u_cpu = M.forward(net.params().astype(np.float64), X[keep].astype(np.float64), graph, nlayers=4, emulate_bf16=True)
+    scale = np.abs(u_cpu).max()
+    err = np.abs(u_gpu - u_cpu)
+    # as test_forward_matches_oracle: float32 sums, bfloat16 roundings that fall the other way
+    assert err.max() <= 2e-2 * scale
+    assert np.sqrt((err ** 2).mean()) <= 2e-3 * scale

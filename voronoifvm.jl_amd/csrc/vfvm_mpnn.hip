@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <random>
 #include <vector>
@@ -502,6 +503,172 @@ __global__ void __launch_bounds__(256) k_smooth_step(int64_t n, int64_t C4, cons
   }
 }
 
+// All smoothing steps of a field in one launch, the field resident in LDS: a block takes one
+// sample (FPB = 2 features, interleaved) or one feature of a sample (FPB = 1).  The nodes
+// whose graph row is the grid's most frequent one (four entries with the same neighbour
+// offsets and weights: the inside of a 2D tensor grid) form groups of 64, up to NG per wave,
+// so a wave's offsets and weights are scalars; the other nodes (sides and corners) form at
+// most one further group per wave, whose lanes carry their own entries in registers.  A
+// node's own value stays in a register.  Sums run in entry order as in k_smooth_step, so both
+// give the same bits.
+// Bound: LDS (four reads and a write per node and step, about 64 bytes a cycle with 4-byte
+// and 85 with 8-byte accesses, so two features together cost 1.5 times one).  Pairs of
+// consecutive nodes per lane, with three two-word reads instead of eight one-word ones, took
+// the same time.  Measured on 129 x 129 nodes, with the copies to and from the node-major
+// fields of the launch-per-step form: 0.70 ms instead of 1.85 for one sample, 2.2 ms instead
+// of 9.4 for 512.
+constexpr int CTX_T = 1024;            // threads per block
+constexpr int CTX_W = CTX_T / 64;      // waves per block
+constexpr int64_t CTX_LDS = 160 * 1024;
+constexpr int CTX_D = 4;               // graph entries of a node
+struct CtxGraph {
+  int nmain, nmix;      // groups of main nodes; groups of other nodes (at most CTX_W)
+  int off[CTX_D];       // the main row's neighbour offsets (in nodes) and weights
+  float w[CTX_D];
+  const int32_t *node;  // (nmain + nmix) x 64 nodes; a short group repeats its last node
+                        // (same value, same place)
+  const int32_t *mdeg;  // nmix x 64: entries of the node, then their columns and weights
+  const int32_t *mcol;  // nmix x 64 x CTX_D
+  const float *mw;
+};
+
+template <int FPB>
+struct CtxVal;
+template <>
+struct CtxVal<1> {
+  using T = float;
+  static __device__ __forceinline__ T fma(float w, T y, T a) { return a + w * y; }
+  static __device__ __forceinline__ T half(T y, T a) { return 0.5f * (y + a); }
+  static __device__ __forceinline__ T zero() { return 0.f; }
+};
+template <>
+struct CtxVal<2> {
+  using T = float2;
+  static __device__ __forceinline__ T fma(float w, T y, T a) {
+    a.x += w * y.x;
+    a.y += w * y.y;
+    return a;
+  }
+  static __device__ __forceinline__ T half(T y, T a) { return make_float2(0.5f * (y.x + a.x), 0.5f * (y.y + a.y)); }
+  static __device__ __forceinline__ T zero() { return make_float2(0.f, 0.f); }
+};
+
+// x: rows x 8 features; P: 8 planes of `rows` values, plane 4 c + k = feature c after
+// SMOOTH_STEPS_H[k] steps
+template <int FPB, int NG>
+__global__ void __launch_bounds__(CTX_T) k_context(int64_t n, int64_t rows, CtxGraph G, const float *__restrict__ x,
+                                                   float *__restrict__ P) {
+  using CV = CtxVal<FPB>;
+  using T = typename CV::T;
+  extern __shared__ __attribute__((aligned(16))) unsigned char ctx_lds[];
+  T *Y = reinterpret_cast<T *>(ctx_lds);
+  const int64_t smp = FPB == 2 ? blockIdx.x : blockIdx.x >> 1;
+  const int c0 = FPB == 2 ? 0 : blockIdx.x & 1;
+  const float *xs = x + smp * n * NFEAT;
+  for (int i = threadIdx.x; i < (int)n; i += CTX_T) {
+    if constexpr (FPB == 2)
+      Y[i] = make_float2(xs[(int64_t)i * NFEAT + SMOOTH_SRC[0]], xs[(int64_t)i * NFEAT + SMOOTH_SRC[1]]);
+    else
+      Y[i] = xs[(int64_t)i * NFEAT + (c0 == 0 ? SMOOTH_SRC[0] : SMOOTH_SRC[1])];
+  }
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // main groups w, w + CTX_W, ...: every wave has as many, or one more
+  int cnt = __builtin_amdgcn_readfirstlane(w < G.nmain ? (G.nmain - w + CTX_W - 1) / CTX_W : 0);
+  uint32_t nd[(NG + 1) / 2];  // the lane's nodes in them, as pairs of 16 bits
+#pragma unroll
+  for (int q = 0; q < NG; q++) {
+    const uint32_t v = q < cnt ? (uint32_t)G.node[(w + q * CTX_W) * 64 + lane] : 0;
+    nd[q / 2] = q % 2 ? nd[q / 2] | (v << 16) : v;
+  }
+  auto node = [&](int q) -> int { return q % 2 ? (int)(nd[q / 2] >> 16) : (int)(nd[q / 2] & 0xffffu); };
+  // the wave's group of other nodes
+  const bool mix = w < G.nmix;
+  int mnode = 0, mdeg = 0, mcol[CTX_D] = {0, 0, 0, 0};
+  float mw[CTX_D] = {0.f, 0.f, 0.f, 0.f};
+  if (mix) {
+    const int k = w * 64 + lane;
+    mnode = G.node[(int64_t)G.nmain * 64 + k];
+    mdeg = G.mdeg[k];
+#pragma unroll
+    for (int e = 0; e < CTX_D; e++) {
+      mcol[e] = G.mcol[k * CTX_D + e];
+      mw[e] = G.mw[k * CTX_D + e];
+    }
+  }
+  const int o0 = G.off[0], o1 = G.off[1], o2 = G.off[2], o3 = G.off[3];
+  const float w0 = G.w[0], w1 = G.w[1], w2 = G.w[2], w3 = G.w[3];
+  __syncthreads();
+  T nv[NG], mv = CV::zero();
+#pragma unroll
+  for (int q = 0; q < NG; q++) nv[q] = q < cnt ? Y[node(q)] : CV::zero();
+  if (mix) mv = Y[mnode];
+  int snap = 0;
+  for (int step = 1; step <= SMOOTH_STEPS_H[3]; step++) {
+    // hides that cnt is loop-invariant (the compiler would keep a mask per group in scalar
+    // registers), and the node numbers where the addresses of every group would not fit the
+    // vector registers: they are then formed again in each step.  The branch on cnt also
+    // keeps the compiler from issuing the loads of all groups at once, which spills (without
+    // it, 512 samples of 129 x 129 nodes took 12 ms instead of 2.2).
+    asm volatile("" : "+s"(cnt));
+    if constexpr (NG * FPB > 16) {
+#pragma unroll
+      for (int q = 0; q < (NG + 1) / 2; q++) asm volatile("" : "+v"(nd[q]));
+    }
+#pragma unroll
+    for (int q = 0; q < NG; q++)
+      if (q < cnt) {  // wave-uniform
+        const int i = node(q);
+        const T y0 = Y[i + o0], y1 = Y[i + o1], y2 = Y[i + o2], y3 = Y[i + o3];
+        T acc = CV::fma(w0, y0, CV::zero());
+        acc = CV::fma(w1, y1, acc);
+        acc = CV::fma(w2, y2, acc);
+        acc = CV::fma(w3, y3, acc);
+        nv[q] = CV::half(nv[q], acc);
+      }
+    if (mix) {
+      T acc = CV::zero();
+#pragma unroll
+      for (int e = 0; e < CTX_D; e++) {
+        const T t = CV::fma(mw[e], Y[mcol[e]], acc);
+        if (e < mdeg) acc = t;
+      }
+      mv = CV::half(mv, acc);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NG; q++)
+      if (q < cnt) Y[node(q)] = nv[q];
+    if (mix) Y[mnode] = mv;
+    if (step == SMOOTH_STEPS_H[snap]) {
+      float *o = P + (int64_t)(4 * c0 + snap) * rows + smp * n;
+      auto put = [&](int i, T v) {
+        if constexpr (FPB == 2) {
+          o[i] = v.x;
+          o[4 * rows + i] = v.y;
+        } else {
+          o[i] = v;
+        }
+      };
+#pragma unroll
+      for (int q = 0; q < NG; q++)
+        if (q < cnt) put(node(q), nv[q]);
+      if (mix) put(mnode, mv);
+      snap++;
+    }
+    __syncthreads();
+  }
+}
+
+// x16 = [x, P]: the network input from the features and the context planes
+__global__ void k_pack16(int64_t rows, const float *__restrict__ x, const float *__restrict__ P,
+                         float *__restrict__ x16) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= rows * KPAD) return;
+  const int64_t r = q / KPAD;
+  const int k = (int)(q % KPAD);
+  x16[q] = k < NFEAT ? x[r * NFEAT + k] : P[(int64_t)(k - NFEAT) * rows + r];
+}
+
 // u_r = h_L[r] . wd + bd (one wave per row); optional loss: du = 2 (u - t) / count,
 // dh = du wd, per-block partials of sum (u-t)^2, sum du h (64) and sum du
 __global__ void __launch_bounds__(TB) k_decode(int64_t rows, const float *__restrict__ hf, const float *__restrict__ wd,
@@ -611,6 +778,10 @@ struct vfvm_mpnn {
   // graph
   DevBuf<int32_t> gptr, gcol;
   DevBuf<float> gw, gwt;
+  // the graph as k_context takes it (nmain 0: it does not)
+  CtxGraph ctxg{};
+  DevBuf<int32_t> ctx_node, ctx_mdeg, ctx_mcol;
+  DevBuf<float> ctx_mw, planes;
   // parameters
   DevBuf<float> theta, grad, adam_m, adam_v;
   int64_t adam_t = 0;
@@ -698,9 +869,126 @@ void copy_in(DevBuf<T> &buf, const T *h, size_t count, hipStream_t st) {
   VFVM_HIP_CHECK(hipStreamSynchronize(st));
 }
 
+// The node groups of k_context: taken where the most frequent graph row has CTX_D entries, no
+// row has more, and the nodes with other rows fit one group per wave.  That holds for the 2D
+// tensor grids that fit the LDS (up to 202 x 202 nodes); unstructured and 3D grids keep one
+// launch per step.
+void build_context_groups(vfvm_mpnn &m, const std::vector<int32_t> &ptr, const std::vector<int32_t> &col,
+                          const std::vector<float> &w) {
+  m.ctxg.nmain = 0;
+  if (m.n < 1 || m.n * (int64_t)sizeof(float) > CTX_LDS) return;
+  using Row = std::vector<std::pair<int32_t, uint32_t>>;  // offset and weight bits per entry
+  std::map<Row, int64_t> count;
+  auto row_of = [&](int64_t i) {
+    Row row;
+    for (int32_t k = ptr[i]; k < ptr[i + 1]; k++) {
+      uint32_t bits;
+      std::memcpy(&bits, &w[k], sizeof(bits));
+      row.emplace_back((int32_t)(col[k] - i), bits);
+    }
+    return row;
+  };
+  for (int64_t i = 0; i < m.n; i++) {
+    if (ptr[i + 1] - ptr[i] > CTX_D) return;
+    count[row_of(i)]++;
+    if ((int64_t)count.size() > (int64_t)CTX_T + 1) return;
+  }
+  auto main = count.begin();
+  for (auto it = count.begin(); it != count.end(); ++it)
+    if (it->second > main->second) main = it;
+  const Row &mr = main->first;
+  if ((int)mr.size() != CTX_D || m.n - main->second > (int64_t)CTX_T) return;
+  std::vector<int32_t> node, rest;
+  for (int64_t i = 0; i < m.n; i++) (row_of(i) == mr ? node : rest).push_back((int32_t)i);
+  while (node.size() % 64) node.push_back(node.back());
+  const int nmain = (int)(node.size() / 64);
+  while (rest.size() % 64) rest.push_back(rest.back());
+  const int nmix = (int)(rest.size() / 64);
+  std::vector<int32_t> mdeg(rest.size()), mcol(rest.size() * CTX_D);
+  std::vector<float> mw(rest.size() * CTX_D, 0.f);
+  for (size_t k = 0; k < rest.size(); k++) {
+    const int32_t i = rest[k];
+    mdeg[k] = ptr[i + 1] - ptr[i];
+    for (int e = 0; e < CTX_D; e++) mcol[k * CTX_D + e] = i;  // absent entries read the node itself
+    for (int32_t q = ptr[i]; q < ptr[i + 1]; q++) {
+      mcol[k * CTX_D + (q - ptr[i])] = col[q];
+      mw[k * CTX_D + (q - ptr[i])] = w[q];
+    }
+  }
+  node.insert(node.end(), rest.begin(), rest.end());
+  hipStream_t st = m.ctx->stream;
+  m.ctx_node.upload(node, st);
+  if (nmix) {
+    m.ctx_mdeg.upload(mdeg, st);
+    m.ctx_mcol.upload(mcol, st);
+    m.ctx_mw.upload(mw, st);
+  }
+  CtxGraph &g = m.ctxg;
+  for (int e = 0; e < CTX_D; e++) {
+    g.off[e] = mr[e].first;
+    std::memcpy(&g.w[e], &mr[e].second, sizeof(float));
+  }
+  g.node = m.ctx_node.p;
+  g.mdeg = m.ctx_mdeg.p;
+  g.mcol = m.ctx_mcol.p;
+  g.mw = m.ctx_mw.p;
+  g.nmix = nmix;
+  g.nmain = nmain;
+}
+
+// The context planes of `ns` samples into m.planes, or false where k_context does not take
+// the graph.  Both features of a sample in one block once that gives every CU a block (256
+// CUs), while both fit the LDS.
+bool context_planes(vfvm_mpnn &m, const float *x, int64_t ns) {
+  if (m.ctxg.nmain == 0) return false;
+  hipStream_t st = m.ctx->stream;
+  const int64_t rows = ns * m.n;
+  const bool two = 2 * ns > 256 && m.n * (int64_t)sizeof(float2) <= CTX_LDS;
+  if (m.planes.n < (size_t)(rows * 8)) m.planes.alloc((size_t)(rows * 8));
+  auto launch = [&](auto fpb, auto ng) {
+    constexpr int FPB = decltype(fpb)::value, NG = decltype(ng)::value;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_context<FPB, NG>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)CTX_LDS);
+    VFVM_HIP_CHECK(attr);
+    hipLaunchKernelGGL((k_context<FPB, NG>), dim3((unsigned)(FPB == 2 ? ns : 2 * ns)), dim3(CTX_T),
+                       (size_t)m.n * sizeof(float) * FPB, st, m.n, rows, m.ctxg, x, m.planes.p);
+  };
+  // registers grow with NG: the smallest that holds the groups of a wave
+  const int need = (m.ctxg.nmain + CTX_W - 1) / CTX_W;
+  auto go = [&](auto ng) {
+    if constexpr (decltype(ng)::value <= 20) {  // both features: at most 20480 nodes
+      if (two) {
+        launch(std::integral_constant<int, 2>(), ng);
+        return;
+      }
+    }
+    launch(std::integral_constant<int, 1>(), ng);
+  };
+  if (need <= 5)
+    go(std::integral_constant<int, 5>());
+  else if (need <= 10)
+    go(std::integral_constant<int, 10>());
+  else if (need <= 16)
+    go(std::integral_constant<int, 16>());
+  else if (need <= 20)
+    go(std::integral_constant<int, 20>());
+  else if (need <= 30)
+    go(std::integral_constant<int, 30>());
+  else
+    go(std::integral_constant<int, 40>());
+  VFVM_HIP_CHECK(hipGetLastError());
+  return true;
+}
+
 // network input of `ns` samples: x16 = [x (8 features), smoothed context (8 channels)]
 void expand(vfvm_mpnn &m, const float *x, float *x16, int64_t ns) {
   hipStream_t st = m.ctx->stream;
+  if (context_planes(m, x, ns)) {
+    hipLaunchKernelGGL(k_pack16, dim3(nb(ns * m.n * KPAD, 256)), dim3(256), 0, st, ns * m.n, x,
+                       (const float *)m.planes.p, x16);
+    VFVM_HIP_CHECK(hipGetLastError());
+    return;
+  }
   const int64_t rows = ns * m.n, Cs = (2 * ns + 3) / 4 * 4, C4 = Cs / 4;
   hipLaunchKernelGGL(k_expand_copy, dim3(nb(rows * KPAD, 256)), dim3(256), 0, st, rows, x, x16);
   m.sm0.alloc((size_t)std::max<int64_t>(m.n * Cs, (int64_t)m.sm0.n));
@@ -930,6 +1218,7 @@ int vfvm_mpnn_create(vfvm_sys *sys, int nlayers, int width, uint64_t seed, vfvm_
     m->gcol.upload(col.empty() ? std::vector<int32_t>{0} : col, st);
     m->gw.upload(w.empty() ? std::vector<float>{0.f} : w, st);
     m->gwt.upload(wt.empty() ? std::vector<float>{0.f} : wt, st);
+    build_context_groups(*m, ptr, col, w);
     // parameter layout and He-uniform initialisation
     size_t p = 0;
     m->off_We = p;
