@@ -213,3 +213,29 @@ def test_testfunction_integral_matches_oracle_and_closed_form():
     Ito = float(T @ Ft)
     _print("transient integral", It, "oracle", Ito)
     assert abs(It - Ito) <= 1e-12 * abs(Ito) and abs(It - I) > 1e-3
+
+
+@pytest.mark.parametrize("shape", [(47, 47), (61, 37), (13, 13, 13)])
+def test_impedance_multigrid_groups_match_oracle(shape):
+    """scalar systems from 2048 unknowns on: groups of frequencies preconditioned by a
+    multigrid cycle of J + sigma M.  Frequencies out of order, repeated, negative and zero;
+    more in one decade than a group holds; and far above the grid's own (the storage term
+    then dominates)."""
+    _print("case impedance multigrid", shape)
+    axes = [np.linspace(0.0, 1.0, m) ** (1.0 if k == 0 else 1.3) for k, m in enumerate(shape)]
+    g = simplexgrid(*axes)
+    sys, osys, ph = _problem(g, D=0.7, R=1.5, excited=4, meas=2)
+    rng = np.random.default_rng(3)
+    om = np.concatenate([rng.permutation(1.0 * 1.03 ** np.arange(70)), [5.0, 5.0, -5.0, 0.0, 1e-3, 40.0]])
+    _, _, ds, dt, Z, isys = _gpu(sys, om, excited=4, meas=2)
+    assert isys.iterations.max() < 40, isys.iterations  # the Jacobi form takes 60 and more
+    pick = np.array([0, 11, 69, 70, 72, 73, 74, 75])
+    _, _, dso, dto, Zo, _ = _oracle(g, osys, ph, om[pick], excited=4, meas=2)
+    err = np.abs(Z[pick] - Zo) / np.abs(Zo)
+    _print("max rel err vs oracle", err.max())
+    assert err.max() <= ZTOL
+    assert Z[70] == Z[71] and abs(Z[72] - np.conj(Z[70])) <= ZTOL * abs(Z[70])
+    far = [-3.0, 1e4, 1e7]
+    _, _, _, _, _, UZo = _oracle(g, osys, ph, far, excited=4, meas=2)
+    for w, ref in zip(far, UZo):
+        assert _rel(isys.solve(w), ref) <= ZTOL

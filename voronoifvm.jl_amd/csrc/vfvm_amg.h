@@ -90,7 +90,7 @@ struct AmgPattern {
     std::vector<int32_t> gptr, gr, ga, gp;
   };
   std::vector<Level> lv;  // lv.back() is the coarsest level
-  void build(int64_t n, const int32_t *rowptr, const int32_t *colind);
+  void build(int64_t n, const int32_t *rowptr, const int32_t *colind, bool recipes = true);
 };
 
 // Standard aggregation on the pattern graph without its diagonal; returns the number of
@@ -112,8 +112,10 @@ class Amg {
 
   // Symbolic setup.  members: the owner's members in order (their level-0 rows are the
   // owner's rows, concatenated); row_inst0: the owner's row -> member map on the device
-  // (nullptr: one member).  Members with equal patterns share the host work.
-  void build(const std::vector<AmgMember> &members, const int32_t *row_inst0, hipStream_t s);
+  // (nullptr: one member).  Members with equal patterns share the host work.  csr_only: for
+  // apply_columns alone, without the SELL-64 matrices and the Galerkin recipes (more than
+  // half of the host work).
+  void build(const std::vector<AmgMember> &members, const int32_t *row_inst0, hipStream_t s, bool csr_only = false);
   bool built() const { return nlev > 0; }
   // Numeric setup from the owner's FP64 Jacobian J (global CSR rowptr / colind, diagonal
   // positions dofdiag) and row scaling: the hierarchy of Ahat = diag(rowscale) J.
@@ -138,6 +140,11 @@ class Amg {
   // it ran on
   template <class V>
   void apply(const V *y, V *z, const KState *st, int skip_half, hipStream_t s, KernelProbe *probe = nullptr);
+  // The same cycle in FP64 for `cols` complex right-hand sides of a single-member hierarchy,
+  // interleaved: value of row i and column w at i * cols + w.  z must not alias y.  Columns
+  // with skip[w] set are left alone (their part of z is not written).
+  void apply_columns(const double2 *y, double2 *z, int cols, const int32_t *rowptr, const int32_t *colind,
+                     const int32_t *skip, hipStream_t s);
   // allocates apply's work vectors of precision V (before a stream capture of apply)
   template <class V>
   void reserve() {
@@ -184,7 +191,7 @@ class Amg {
     // the matrices of the cycle
     SellMat A, P, R;
     // coarsening members: (member, first row, end row) for the omega reduction
-    int64_t ncm = 0;
+    int64_t ncm = 0, nmax = 0;  // and the most rows of one
     DevBuf<int32_t> cm;
     DevBuf<int64_t> cb, ce;
     // Galerkin recipe per distinct pattern of the coarsening members: the pattern's
@@ -210,6 +217,7 @@ class Amg {
     // work vectors of the apply (b: right-hand side, x: iterate, r: residual / solution)
     DevBuf<double> b64, x64, rv64;
     DevBuf<float> b32, x32, rv32;
+    DevBuf<double2> cb2, cx2, cr2;  // of apply_columns
   };
   template <class V>
   void work(Lev &L, V *&b, V *&x, V *&r) {
@@ -237,6 +245,8 @@ class Amg {
   std::vector<int32_t> pid;  // member -> pattern
   std::vector<Lev> lev;
   int64_t nnz0 = 0;
+  bool csr_only = false;
+  DevBuf<unsigned long long> omax;  // per member: bits of the largest row sum (k_amg_omega)
   // coarse tail: first level, its members, and the per-level device tables per precision
   int lt = 0;
   int64_t ntail = 0;

@@ -41,14 +41,16 @@ __global__ void __launch_bounds__(AB) k_amg_scale0(int64_t n, const int32_t *__r
 }
 
 // omega = (4/3) / rho(D^-1 A) per listed member, rho bounded by the largest row sum of
-// |D^-1 A| (Gershgorin); one block per member
-__global__ void __launch_bounds__(AB) k_amg_omega(const int32_t *__restrict__ cm, const int64_t *__restrict__ cb,
-                                                  const int64_t *__restrict__ ce, const int32_t *__restrict__ arp,
-                                                  const int32_t *__restrict__ adp, const double *__restrict__ aval,
-                                                  double *__restrict__ w) {
-  const int k = blockIdx.x;
+// |D^-1 A| (Gershgorin).  Block (b, k) takes every gridDim.x-th run of rows of member k and
+// merges its largest sum into mx[k] (bits of a non-negative double order as integers, so the
+// result does not depend on the order of the blocks); k_amg_omega_fin forms omega.  One block
+// per member took 325 us on 263,169 rows, waiting for one CU's loads.
+__global__ void __launch_bounds__(AB) k_amg_omega(const int64_t *__restrict__ cb, const int64_t *__restrict__ ce,
+                                                  const int32_t *__restrict__ arp, const int32_t *__restrict__ adp,
+                                                  const double *__restrict__ aval, unsigned long long *mx_out) {
+  const int k = blockIdx.y;
   double mx = 0.0;
-  for (int64_t i = cb[k] + threadIdx.x; i < ce[k]; i += AB) {
+  for (int64_t i = cb[k] + (int64_t)blockIdx.x * AB + threadIdx.x; i < ce[k]; i += (int64_t)gridDim.x * AB) {
     const double d = fabs(aval[adp[i]]);
     double s = 0.0;
     for (int32_t q = arp[i]; q < arp[i + 1]; q++) s += fabs(aval[q]);
@@ -56,14 +58,16 @@ __global__ void __launch_bounds__(AB) k_amg_omega(const int32_t *__restrict__ cm
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-  __shared__ double sh[AB / 64];
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double r = 0.0;
-    for (int j = 0; j < AB / 64; j++) r = fmax(r, sh[j]);
-    w[cm[k]] = r > 0.0 ? (4.0 / 3.0) / r : 0.0;
-  }
+  if ((threadIdx.x & 63) == 0 && mx > 0.0) atomicMax(mx_out + k, (unsigned long long)__double_as_longlong(mx));
+}
+
+__global__ void __launch_bounds__(AB) k_amg_omega_fin(int64_t ncm, const int32_t *__restrict__ cm,
+                                                      unsigned long long *__restrict__ mx, double *__restrict__ w) {
+  const int64_t k = (int64_t)blockIdx.x * AB + threadIdx.x;
+  if (k >= ncm) return;
+  const double r = __longlong_as_double((long long)mx[k]);
+  mx[k] = 0ull;  // for the next level
+  w[cm[k]] = r > 0.0 ? (4.0 / 3.0) / r : 0.0;
 }
 
 // P = (I - omega D^-1 A) T, one thread per row of a coarsening member: the row of A T is
@@ -87,20 +91,12 @@ __global__ void __launch_bounds__(AB) k_amg_prol(int64_t n, const int32_t *__res
   pval[tpos[i]] += tval[i];
 }
 
-// position of key in the sorted c[lo, hi) (key present)
-__device__ __forceinline__ int32_t amg_find(const int32_t *__restrict__ c, int32_t lo, int32_t hi, int32_t key) {
-  while (hi - lo > 1) {
-    const int32_t mid = (lo + hi) >> 1;
-    if (c[mid] <= key)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
-// Galerkin product Ac = P^T A P, one thread per coarse row I: the sum over the fine rows i
-// of column I of P (the rows of P^T) of P[i,I] A[i,k] P[k,J], added into Ac row I's slot J
+// Galerkin product Ac = P^T A P, one wave per coarse row I, one lane per entry of the row
+// (64 at a time): the sum over the fine rows i of column I of P (the rows of P^T) of
+// P[i,I] A[i,k] P[k,J].  The walk over (i, k, J) is the same for all lanes (scalar loads), a
+// lane keeps the terms of its own column J.  One thread per coarse row with a search and a
+// read-modify-write in memory per term took about 1 ms on 66,049 fine rows, mostly waiting;
+// the sums run in the same order.
 __global__ void __launch_bounds__(AB) k_amg_rap(int64_t nc, const int32_t *__restrict__ rrp,
                                                 const int32_t *__restrict__ rci, const int32_t *__restrict__ r2p,
                                                 const int32_t *__restrict__ arp, const int32_t *__restrict__ aci,
@@ -108,18 +104,24 @@ __global__ void __launch_bounds__(AB) k_amg_rap(int64_t nc, const int32_t *__res
                                                 const int32_t *__restrict__ pci, const double *__restrict__ pval,
                                                 const int32_t *__restrict__ crp, const int32_t *__restrict__ cci,
                                                 double *__restrict__ cval) {
-  const int64_t I = (int64_t)blockIdx.x * AB + threadIdx.x;
+  const int32_t I = __builtin_amdgcn_readfirstlane((int32_t)(blockIdx.x * (AB / 64) + (threadIdx.x >> 6)));
   if (I >= nc) return;
-  const int32_t c0 = crp[I], c1 = crp[I + 1];
-  for (int32_t c = c0; c < c1; c++) cval[c] = 0.0;
-  for (int32_t q = rrp[I]; q < rrp[I + 1]; q++) {
-    const int32_t i = rci[q];
-    const double pI = pval[r2p[q]];
-    for (int32_t a = arp[i]; a < arp[i + 1]; a++) {
-      const int32_t k = aci[a];
-      const double f = pI * aval[a];
-      for (int32_t b = prp[k]; b < prp[k + 1]; b++) cval[amg_find(cci, c0, c1, pci[b])] += f * pval[b];
+  const int32_t c1 = crp[I + 1], q0 = rrp[I], q1 = rrp[I + 1];
+  for (int32_t c = crp[I]; c < c1; c += 64) {
+    const int32_t mine = c + (int32_t)(threadIdx.x & 63);
+    const int32_t J = mine < c1 ? cci[mine] : -1;
+    double acc = 0.0;
+    for (int32_t q = q0; q < q1; q++) {
+      const int32_t i = rci[q], a1 = arp[i + 1];
+      const double pI = pval[r2p[q]];
+      for (int32_t a = arp[i]; a < a1; a++) {
+        const int32_t k = aci[a], b1 = prp[k + 1];
+        const double f = pI * aval[a];
+        for (int32_t b = prp[k]; b < b1; b++)
+          if (pci[b] == J) acc += f * pval[b];
+      }
     }
+    if (mine < c1) cval[mine] = acc;
   }
 }
 
@@ -456,6 +458,111 @@ __global__ void __launch_bounds__(AB) k_amg_dense_apply(const int32_t *__restric
   }
 }
 
+// ---------------------------------------------------------------- interleaved columns
+
+// The V-cycle on `cols` complex vectors at once, interleaved per row: thread (row, column),
+// the columns of a row side by side, so a matrix entry is read once for all of them (one
+// broadcast per row and wave) and every vector access is contiguous.  256 / cols rows per
+// block.  Bound: the vectors' bytes on the fine levels, launches on the coarse ones.
+struct ColRow {
+  int64_t i;  // row (n when there is none)
+  int w;
+};
+__device__ __forceinline__ ColRow col_row(int64_t n, int cols, const int32_t *skip) {
+  const int rpb = AB / cols, r = (int)threadIdx.x / cols;
+  ColRow c;
+  c.w = (int)threadIdx.x - r * cols;
+  c.i = (int64_t)blockIdx.x * rpb + r;
+  if (r >= rpb || c.i >= n || skip[c.w]) c.i = n;
+  return c;
+}
+
+// sum_q a(q) x[col(q)] over the entries q0 <= q < q1
+template <class FA, class FC>
+__device__ __forceinline__ double2 col_sum(int32_t q0, int32_t q1, FA &&a, FC &&col, const double2 *__restrict__ x,
+                                           int cols, int w) {
+  double2 s = make_double2(0.0, 0.0);
+#pragma unroll 4
+  for (int32_t q = q0; q < q1; q++) {
+    const double v = a(q);
+    const double2 xv = x[(int64_t)col(q) * cols + w];
+    s.x += v * xv.x;
+    s.y += v * xv.y;
+  }
+  return s;
+}
+
+// r = b - A (w D^-1 b)
+__global__ void __launch_bounds__(AB) k_amgc_down(int64_t n, int cols, const int32_t *__restrict__ rp,
+                                                  const int32_t *__restrict__ ci, const double *__restrict__ av,
+                                                  const double *__restrict__ dinv, const double *__restrict__ wm,
+                                                  const double2 *__restrict__ b, double2 *__restrict__ r,
+                                                  const int32_t *__restrict__ skip) {
+  const ColRow c = col_row(n, cols, skip);
+  if (c.i >= n) return;
+  const double2 s = col_sum(rp[c.i], rp[c.i + 1], [&](int32_t q) { return dinv ? av[q] * dinv[ci[q]] : av[q]; },
+                            [&](int32_t q) { return ci[q]; }, b, cols, c.w);
+  const double om = wm[0];
+  const double2 bi = b[c.i * cols + c.w];
+  r[c.i * cols + c.w] = make_double2(bi.x - om * s.x, bi.y - om * s.y);
+}
+
+// bc = P^T r
+__global__ void __launch_bounds__(AB) k_amgc_restrict(int64_t nc, int cols, const int32_t *__restrict__ rrp,
+                                                      const int32_t *__restrict__ rci, const int32_t *__restrict__ r2p,
+                                                      const double *__restrict__ pval, const double2 *__restrict__ r,
+                                                      double2 *__restrict__ bc, const int32_t *__restrict__ skip) {
+  const ColRow c = col_row(nc, cols, skip);
+  if (c.i >= nc) return;
+  bc[c.i * cols + c.w] = col_sum(rrp[c.i], rrp[c.i + 1], [&](int32_t q) { return pval[r2p[q]]; },
+                                 [&](int32_t q) { return rci[q]; }, r, cols, c.w);
+}
+
+// x = w D^-1 b + P xc
+__global__ void __launch_bounds__(AB) k_amgc_prolong(int64_t n, int cols, const int32_t *__restrict__ prp,
+                                                     const int32_t *__restrict__ pci, const double *__restrict__ pval,
+                                                     const double *__restrict__ dinv, const double *__restrict__ wm,
+                                                     const double2 *__restrict__ b, const double2 *__restrict__ xc,
+                                                     double2 *__restrict__ x, const int32_t *__restrict__ skip) {
+  const ColRow c = col_row(n, cols, skip);
+  if (c.i >= n) return;
+  const double2 s = col_sum(prp[c.i], prp[c.i + 1], [&](int32_t q) { return pval[q]; },
+                            [&](int32_t q) { return pci[q]; }, xc, cols, c.w);
+  const double d = wm[0] * (dinv ? dinv[c.i] : 1.0);
+  const double2 bi = b[c.i * cols + c.w];
+  x[c.i * cols + c.w] = make_double2(d * bi.x + s.x, d * bi.y + s.y);
+}
+
+// out = x + w D^-1 (b - A x); x null: out = w D^-1 b
+__global__ void __launch_bounds__(AB) k_amgc_sweep(int64_t n, int cols, const int32_t *__restrict__ rp,
+                                                   const int32_t *__restrict__ ci, const double *__restrict__ av,
+                                                   const double *__restrict__ dinv, const double *__restrict__ wm,
+                                                   const double2 *__restrict__ b, const double2 *__restrict__ x,
+                                                   double2 *__restrict__ out, const int32_t *__restrict__ skip) {
+  const ColRow c = col_row(n, cols, skip);
+  if (c.i >= n) return;
+  const double d = wm[0] * (dinv ? dinv[c.i] : 1.0);
+  const double2 bi = b[c.i * cols + c.w];
+  if (!x) {
+    out[c.i * cols + c.w] = make_double2(d * bi.x, d * bi.y);
+    return;
+  }
+  const double2 s = col_sum(rp[c.i], rp[c.i + 1], [&](int32_t q) { return av[q]; }, [&](int32_t q) { return ci[q]; },
+                            x, cols, c.w);
+  const double2 xi = x[c.i * cols + c.w];
+  out[c.i * cols + c.w] = make_double2(xi.x + d * (bi.x - s.x), xi.y + d * (bi.y - s.y));
+}
+
+// out = Ac^-1 b on the coarsest level
+__global__ void __launch_bounds__(AB) k_amgc_dense(int64_t n, int cols, const double *__restrict__ inv,
+                                                   const double2 *__restrict__ b, double2 *__restrict__ out,
+                                                   const int32_t *__restrict__ skip) {
+  const ColRow c = col_row(n, cols, skip);
+  if (c.i >= n) return;
+  out[c.i * cols + c.w] = col_sum(0, (int32_t)n, [&](int32_t q) { return inv[c.i * n + q]; },
+                                  [&](int32_t q) { return q; }, b, cols, c.w);
+}
+
 uint64_t pattern_hash(int64_t n, const int32_t *rp, const int32_t *ci) {
   uint64_t h = 1469598103934665603ull;
   auto mix = [&](uint64_t v) {
@@ -510,7 +617,7 @@ int64_t amg_aggregate(int64_t n, const int32_t *rp, const int32_t *ci, std::vect
   return na;
 }
 
-void AmgPattern::build(int64_t n, const int32_t *rowptr, const int32_t *colind) {
+void AmgPattern::build(int64_t n, const int32_t *rowptr, const int32_t *colind, bool want_recipes) {
   lv.clear();
   lv.emplace_back();
   {
@@ -610,8 +717,8 @@ void AmgPattern::build(int64_t n, const int32_t *rowptr, const int32_t *colind) 
         for (int32_t q = C.arp[I]; q < C.arp[I + 1]; q++)
           if (C.aci[q] == I) C.adp[I] = q;
       // Galerkin recipe: count the products of every coarse entry, then list them
-      int64_t ntrip = 0;
-      for (int64_t I = 0; I < na; I++)
+      int64_t ntrip = want_recipes ? 0 : Amg::MAX_TRIPLES + 1;
+      for (int64_t I = 0; I < na && want_recipes; I++)
         for (int32_t q = L.rrp[I]; q < L.rrp[I + 1]; q++) {
           const int32_t i = L.rci[q];
           for (int32_t a = L.arp[i]; a < L.arp[i + 1]; a++) ntrip += L.prp[L.aci[a] + 1] - L.prp[L.aci[a]];
@@ -730,7 +837,8 @@ void Amg::build_sell(int l, int kind, SellMat &M, hipStream_t s) {
   VFVM_HIP_CHECK(hipMemsetAsync(M.v16.p, 0, sizeof(_Float16) * M.v16.n, s));
 }
 
-void Amg::build(const std::vector<AmgMember> &members, const int32_t *row_inst0, hipStream_t s) {
+void Amg::build(const std::vector<AmgMember> &members, const int32_t *row_inst0, hipStream_t s, bool columns) {
+  csr_only = columns;
   nsys = (int64_t)members.size();
   patterns.clear();
   pid.assign((size_t)nsys, -1);
@@ -753,7 +861,7 @@ void Amg::build(const std::vector<AmgMember> &members, const int32_t *row_inst0,
     }
     if (pid[m] < 0) {
       patterns.emplace_back();
-      patterns.back().build(M.n, M.rowptr, M.colind);
+      patterns.back().build(M.n, M.rowptr, M.colind, !csr_only);
       pid[m] = (int32_t)patterns.size() - 1;
       cand.push_back(pid[m]);
     }
@@ -799,6 +907,7 @@ void Amg::build(const std::vector<AmgMember> &members, const int32_t *row_inst0,
       ms[2 * m + 1] = members[m].rowptr[members[m].n];
     }
     msize0.upload(ms, s);
+    omax.upload(std::vector<unsigned long long>((size_t)nsys, 0ull), s);
   }
   for (int l = 0; l < nlev; l++) {
     Lev &L = lev[l];
@@ -888,7 +997,7 @@ void Amg::build(const std::vector<AmgMember> &members, const int32_t *row_inst0,
       L.inst_p = row_inst0;
       L.aval.alloc((size_t)L.nnzA);
     }
-    build_sell(l, 0, L.A, s);
+    if (!csr_only) build_sell(l, 0, L.A, s);
     {
       std::vector<int32_t> hm(L.hmode.begin(), L.hmode.end());
       L.mode.upload(hm, s);
@@ -896,6 +1005,7 @@ void Amg::build(const std::vector<AmgMember> &members, const int32_t *row_inst0,
     L.w.alloc((size_t)nsys);
     VFVM_HIP_CHECK(hipMemsetAsync(L.w.p, 0, sizeof(double) * nsys, s));
     L.ncm = (int64_t)cm.size();
+    for (size_t k = 0; k < cm.size(); k++) L.nmax = std::max(L.nmax, ce[k] - cb[k]);
     if (L.ncm) {
       L.cm.upload(cm, s);
       L.cb.upload(cb, s);
@@ -912,8 +1022,10 @@ void Amg::build(const std::vector<AmgMember> &members, const int32_t *row_inst0,
       L.rrp.upload(rrp, s);
       L.rci.upload(rci, s);
       L.r2p.upload(r2p, s);
-      build_sell(l, 1, L.P, s);
-      build_sell(l, 2, L.R, s);
+      if (!csr_only) {
+        build_sell(l, 1, L.P, s);
+        build_sell(l, 2, L.R, s);
+      }
     }
     if (coarsen) {  // Galerkin recipes, one per distinct pattern of the coarsening members
       std::map<int32_t, std::vector<int64_t>> bypat;
@@ -1073,22 +1185,30 @@ void Amg::setup(const int32_t *rowptr, const int32_t *colind, const int32_t *dof
   if (!built()) throw Error(VFVM_ERR_ARG, "AMG: numeric setup before the symbolic one");
   hipLaunchKernelGGL(k_amg_scale0, dim3(agrid(lev[0].n)), dim3(AB), 0, s, lev[0].n, rowptr, rowscale, J,
                      lev[0].aval.p);
-  hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(lev[0].n)), dim3(AB), 0, s, lev[0].n, rowptr,
-                     (const int64_t *)lev[0].A.rbase.p, (const double *)lev[0].aval.p, (const int32_t *)nullptr,
-                     (const double *)nullptr, lev[0].A.v64.p, lev[0].A.v16.p);
+  if (!csr_only)
+    hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(lev[0].n)), dim3(AB), 0, s, lev[0].n, rowptr,
+                       (const int64_t *)lev[0].A.rbase.p, (const double *)lev[0].aval.p, (const int32_t *)nullptr,
+                       (const double *)nullptr, lev[0].A.v64.p, lev[0].A.v16.p);
   for (int l = 0; l < nlev; l++) {
     Lev &L = lev[l];
     const int32_t *arp = l ? L.arp.p : rowptr;
     const int32_t *aci = l ? L.aci.p : colind;
     const int32_t *adp = l ? L.adp.p : dofdiag;
+    for (int64_t k0 = 0; k0 < L.ncm; k0 += 65535) {
+      const int64_t nk = std::min<int64_t>(L.ncm - k0, 65535);
+      // about 1024 blocks, 4 or more rows of the longest member per thread
+      const int64_t nb = std::max<int64_t>(1, std::min<int64_t>((L.nmax + 4 * AB - 1) / (4 * AB), 1024 / nk));
+      hipLaunchKernelGGL(k_amg_omega, dim3((unsigned)nb, (unsigned)nk), dim3(AB), 0, s, L.cb.p + k0, L.ce.p + k0, arp,
+                         adp, L.aval.p, omax.p + k0);
+    }
     if (L.ncm)
-      hipLaunchKernelGGL(k_amg_omega, dim3((unsigned)L.ncm), dim3(AB), 0, s, L.cm.p, L.cb.p, L.ce.p, arp, adp,
-                         L.aval.p, L.w.p);
+      hipLaunchKernelGGL(k_amg_omega_fin, dim3(agrid(L.ncm)), dim3(AB), 0, s, L.ncm, L.cm.p, omax.p, L.w.p);
     if (l > 0) {
       hipLaunchKernelGGL(k_amg_dinv, dim3(agrid(L.n)), dim3(AB), 0, s, L.n, adp, L.aval.p, L.dinv64.p, L.dinv32.p);
-      hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(L.n)), dim3(AB), 0, s, L.n, arp, (const int64_t *)L.A.rbase.p,
-                         (const double *)L.aval.p, (const int32_t *)nullptr, (const double *)nullptr, L.A.v64.p,
-                         L.A.v16.p);
+      if (!csr_only)
+        hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(L.n)), dim3(AB), 0, s, L.n, arp, (const int64_t *)L.A.rbase.p,
+                           (const double *)L.aval.p, (const int32_t *)nullptr, (const double *)nullptr, L.A.v64.p,
+                           L.A.v16.p);
     }
     if (L.any_coarsen) {
       Lev &C = lev[l + 1];
@@ -1101,15 +1221,17 @@ void Amg::setup(const int32_t *rowptr, const int32_t *colind, const int32_t *dof
                                dim3(AB), 0, s, R.nslot, R.gcnt.p, R.gsb.p, R.gr.p, R.ga.p, R.gp.p, R.maoff.p,
                                R.mpoff.p, R.mcoff.p, m0, L.aval.p, L.pval.p, C.aval.p);
       } else {
-        hipLaunchKernelGGL(k_amg_rap, dim3(agrid(C.n)), dim3(AB), 0, s, C.n, L.rrp.p, L.rci.p, L.r2p.p, arp, aci,
+        hipLaunchKernelGGL(k_amg_rap, dim3((unsigned)((C.n + AB / 64 - 1) / (AB / 64))), dim3(AB), 0, s, C.n, L.rrp.p, L.rci.p, L.r2p.p, arp, aci,
                            L.aval.p, L.prp.p, L.pci.p, L.pval.p, C.arp.p, C.aci.p, C.aval.p);
       }
-      hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(L.n)), dim3(AB), 0, s, L.n, (const int32_t *)L.prp.p,
-                         (const int64_t *)L.P.rbase.p, (const double *)L.pval.p, (const int32_t *)nullptr,
-                         (const double *)nullptr, L.P.v64.p, L.P.v16.p);
-      hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(C.n)), dim3(AB), 0, s, C.n, (const int32_t *)L.rrp.p,
-                         (const int64_t *)L.R.rbase.p, (const double *)L.pval.p, (const int32_t *)L.r2p.p,
-                         (const double *)nullptr, L.R.v64.p, L.R.v16.p);
+      if (!csr_only) {
+        hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(L.n)), dim3(AB), 0, s, L.n, (const int32_t *)L.prp.p,
+                           (const int64_t *)L.P.rbase.p, (const double *)L.pval.p, (const int32_t *)nullptr,
+                           (const double *)nullptr, L.P.v64.p, L.P.v16.p);
+        hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(C.n)), dim3(AB), 0, s, C.n, (const int32_t *)L.rrp.p,
+                           (const int64_t *)L.R.rbase.p, (const double *)L.pval.p, (const int32_t *)L.r2p.p,
+                           (const double *)nullptr, L.R.v64.p, L.R.v16.p);
+      }
     }
     if (L.ndm) {
       const size_t shm = sizeof(double) * (size_t)L.dmax * (size_t)L.dmax;
@@ -1122,7 +1244,7 @@ void Amg::setup(const int32_t *rowptr, const int32_t *colind, const int32_t *dof
 }
 
 void Amg::refresh_fine(const int32_t *rowptr, const double *J, const double *rowscale, bool fp32, hipStream_t s) {
-  if (!built()) throw Error(VFVM_ERR_ARG, "AMG: refresh before the symbolic setup");
+  if (!built() || csr_only) throw Error(VFVM_ERR_ARG, "AMG: refresh before the symbolic setup");
   Lev &L = lev[0];
   hipLaunchKernelGGL(k_amg_to_sell, dim3(agrid(L.n)), dim3(AB), 0, s, L.n, rowptr, (const int64_t *)L.A.rbase.p, J,
                      (const int32_t *)nullptr, rowscale, fp32 ? (double *)nullptr : L.A.v64.p, L.A.v16.p);
@@ -1131,7 +1253,7 @@ void Amg::refresh_fine(const int32_t *rowptr, const double *J, const double *row
 
 template <class V>
 void Amg::apply(const V *y, V *z, const KState *st, int skip_half, hipStream_t s, KernelProbe *probe) {
-  if (!numeric_ready) throw Error(VFVM_ERR_ARG, "AMG: apply before the numeric setup");
+  if (!numeric_ready || csr_only) throw Error(VFVM_ERR_ARG, "AMG: apply before the numeric setup");
   constexpr bool F32 = sizeof(V) == 4;
   std::vector<V *> B((size_t)nlev), X((size_t)nlev), R((size_t)nlev);
   for (int l = 0; l < nlev; l++) work<V>(lev[l], B[l], X[l], R[l]);
@@ -1208,6 +1330,60 @@ void Amg::apply(const V *y, V *z, const KState *st, int skip_half, hipStream_t s
                 probed ? probe->counters(kid) : (unsigned long long *)nullptr, (const int64_t *)msize0.p);
     if (probed) probe->after(kid, s);
   }
+}
+
+void Amg::apply_columns(const double2 *y, double2 *z, int cols, const int32_t *rowptr, const int32_t *colind,
+                        const int32_t *skip, hipStream_t s) {
+  if (!numeric_ready || nsys != 1) throw Error(VFVM_ERR_ARG, "AMG: apply_columns needs one member, set up");
+  if (cols < 1 || cols > AB) throw Error(VFVM_ERR_ARG, "AMG: apply_columns takes 1 to 256 columns");
+  for (int l = 0; l < nlev; l++) {
+    Lev &L = lev[l];
+    const size_t need = (size_t)(L.n * cols);
+    if (L.cx2.n < need) L.cx2.alloc(need);
+    if (l && L.cb2.n < need) L.cb2.alloc(need);
+    if (l && L.cr2.n < need) L.cr2.alloc(need);
+  }
+  auto bof = [&](int l) -> const double2 * { return l ? lev[l].cb2.p : y; };
+  auto rof = [&](int l) -> double2 * { return l ? lev[l].cr2.p : z; };  // residual, then the level's solution
+  auto arp = [&](int l) { return l ? (const int32_t *)lev[l].arp.p : rowptr; };
+  auto aci = [&](int l) { return l ? (const int32_t *)lev[l].aci.p : colind; };
+  auto dinv = [&](int l) { return l ? (const double *)lev[l].dinv64.p : (const double *)nullptr; };
+  const int rpb = AB / cols;
+  auto grid = [&](int64_t n) { return dim3((unsigned)((n + rpb - 1) / rpb)); };
+  int l = 0;
+  for (; lev[l].hmode[0] == MODE_COARSEN; l++) {
+    Lev &L = lev[l];
+    hipLaunchKernelGGL(k_amgc_down, grid(L.n), dim3(AB), 0, s, L.n, cols, arp(l), aci(l), (const double *)L.aval.p,
+                       dinv(l), (const double *)L.w.p, bof(l), rof(l), skip);
+    hipLaunchKernelGGL(k_amgc_restrict, grid(L.nc), dim3(AB), 0, s, L.nc, cols, (const int32_t *)L.rrp.p,
+                       (const int32_t *)L.rci.p, (const int32_t *)L.r2p.p, (const double *)L.pval.p,
+                       (const double2 *)rof(l), lev[l + 1].cb2.p, skip);
+  }
+  {
+    Lev &L = lev[l];
+    if (L.hmode[0] == MODE_DENSE) {
+      hipLaunchKernelGGL(k_amgc_dense, grid(L.n), dim3(AB), 0, s, L.n, cols, (const double *)L.dinvA64.p, bof(l),
+                         rof(l), skip);
+    } else {  // damped Jacobi from zero, an odd count of sweeps after the first ends in rof(l)
+      const double2 *x = nullptr;
+      double2 *o = L.cx2.p, *t = rof(l);
+      for (int k = 0; k < COARSE_SWEEPS; k++) {
+        hipLaunchKernelGGL(k_amgc_sweep, grid(L.n), dim3(AB), 0, s, L.n, cols, arp(l), aci(l),
+                           (const double *)L.aval.p, dinv(l), (const double *)L.w.p, bof(l), x, o, skip);
+        x = o;
+        std::swap(o, t);
+      }
+    }
+  }
+  for (l = l - 1; l >= 0; l--) {
+    Lev &L = lev[l];
+    hipLaunchKernelGGL(k_amgc_prolong, grid(L.n), dim3(AB), 0, s, L.n, cols, (const int32_t *)L.prp.p,
+                       (const int32_t *)L.pci.p, (const double *)L.pval.p, dinv(l), (const double *)L.w.p, bof(l),
+                       (const double2 *)rof(l + 1), L.cx2.p, skip);
+    hipLaunchKernelGGL(k_amgc_sweep, grid(L.n), dim3(AB), 0, s, L.n, cols, arp(l), aci(l), (const double *)L.aval.p,
+                       dinv(l), (const double *)L.w.p, bof(l), (const double2 *)L.cx2.p, rof(l), skip);
+  }
+  VFVM_HIP_CHECK(hipGetLastError());
 }
 
 template void Amg::apply<float>(const float *, float *, const KState *, int, hipStream_t, KernelProbe *);
