@@ -212,6 +212,8 @@ int natural_levels(int64_t n, const std::vector<int32_t> &rowptr, const std::vec
   return nl;
 }
 
+void build_red_black(vfvm_sys &s, const std::vector<int32_t> &perm, const std::vector<int32_t> &iperm);
+
 void build_ilu(vfvm_sys &s, bool natural) {
   if (s.ilu_built && s.ilu_natural == natural) return;
   s.ilu_built = false;
@@ -279,8 +281,92 @@ void build_ilu(vfvm_sys &s, bool natural) {
   s.ilu.perm = s.d_ilu_perm.p;
   s.ilu.src = s.d_ilu_src.p;
   s.ilu.srcrow = s.d_ilu_srcrow.p;
+  s.ilu.rb = RedBlack();
+  if (!natural) build_red_black(s, perm, iperm);
   s.ilu_built = true;
   s.ilu_natural = natural;
+}
+
+// The two-colour form of the structure (RedBlack, vfvm_linalg.h) where the colouring has two
+// colours; after build_ilu's arrays (perm in colour order).
+void build_red_black(vfvm_sys &s, const std::vector<int32_t> &perm, const std::vector<int32_t> &iperm) {
+  RedBlack &R = s.ilu.rb;
+  R = RedBlack();
+  if (s.ilu.ncolors != 2) return;
+  hipStream_t st = s.ctx->stream;
+  const int32_t nr = s.ilu.cptr[1], n = (int32_t)s.ndof;
+  auto half = [&](int32_t r0, int32_t r1, int32_t c0, int32_t nc, vfvm_sys::RbHalf &D, RedBlack::Half &H,
+                  std::vector<int32_t> *tsrc) -> bool {
+    const int32_t m = r1 - r0;
+    std::vector<int32_t> sptr((size_t)(m + 63) / 64 + 1, 0), col, src, row(perm.begin() + r0, perm.begin() + r1);
+    for (int32_t sl = 0; sl < (m + 63) / 64; sl++) {
+      int32_t w = 1;  // a value slot per row, for the mark of an unusable diagonal
+      for (int32_t i = sl * 64; i < std::min(m, sl * 64 + 64); i++)
+        w = std::max(w, s.rowptr[perm[r0 + i] + 1] - s.rowptr[perm[r0 + i]] - 1);
+      sptr[sl + 1] = sptr[sl] + 64 * w;
+    }
+    const size_t nval = (size_t)sptr.back();
+    col.assign(nval, 0);
+    src.assign(nval, -1);
+    if (tsrc) tsrc->assign(nval, -1);
+    std::vector<int16_t> off(nval, 0);
+    bool fits = true;
+    for (int32_t i = 0; i < (m + 63) / 64 * 64; i++) {
+      const int32_t sl = i / 64, w = (sptr[sl + 1] - sptr[sl]) / 64;
+      int32_t j = 0;
+      // padding: value 0 at a valid column near the row
+      const int32_t self = std::min(i, nc - 1);
+      auto put = [&](int32_t c, int32_t k, int32_t tk) {
+        const size_t q = (size_t)sptr[sl] + (size_t)64 * j + i % 64;
+        col[q] = c;
+        src[q] = k;
+        if (tsrc) (*tsrc)[q] = tk;
+        const int32_t d = c - i;
+        if (d < -32768 || d > 32767)
+          fits = false;
+        else
+          off[q] = (int16_t)d;
+        j++;
+      };
+      if (i < m) {
+        const int32_t r = row[i];
+        for (int32_t k = s.rowptr[r]; k < s.rowptr[r + 1]; k++) {
+          const int32_t c = s.colind[k];
+          if (c == r) continue;
+          if (iperm[c] < c0 || iperm[c] >= c0 + nc) return false;  // a neighbour of its own colour
+          int32_t tk = -1;
+          if (tsrc) {
+            const int32_t *b = s.colind.data() + s.rowptr[c], *e = s.colind.data() + s.rowptr[c + 1];
+            const int32_t *q = std::lower_bound(b, e, r);
+            if (q != e && *q == r) tk = (int32_t)(q - s.colind.data());
+          }
+          put(iperm[c] - c0, k, tk);
+        }
+      }
+      while (j < w) put(self, -1, -1);
+    }
+    D.sptr.upload(sptr, st);
+    D.src.upload(src, st);
+    D.row.upload(row, st);
+    D.col.upload(col, st);
+    D.off.release();
+    if (fits) D.off.upload(off, st);
+    VFVM_HIP_CHECK(hipStreamSynchronize(st));
+    H.nval = (int64_t)nval;
+    H.sptr = D.sptr.p;
+    H.col = D.col.p;
+    H.off = D.off.p;
+    H.src = D.src.p;
+    H.row = D.row.p;
+    return true;
+  };
+  std::vector<int32_t> tsrc;
+  if (!half(0, nr, nr, n - nr, s.d_rb_e, R.e, nullptr) || !half(nr, n, 0, nr, s.d_rb_f, R.f, &tsrc)) return;
+  s.d_rb_tsrc.upload(tsrc, st);
+  VFVM_HIP_CHECK(hipStreamSynchronize(st));
+  R.tsrc = s.d_rb_tsrc.p;
+  R.nb = n - nr;
+  R.nr = nr;
 }
 
 void setup_linear(vfvm_sys &s, const vfvm_control_t &c) {

@@ -96,8 +96,24 @@ __device__ __forceinline__ void run_stage(KState *st, const double *tot) {
   }
 }
 
+// Two-colour form of a multicolour ILU(0) (device pointers): rows in colour order, nr red rows
+// first, and the off-diagonal part of each colour's rows as a SELL-64 matrix over the other
+// colour's rows (numbered from 0 within their colour).
+struct RedBlack {
+  int64_t nr = 0, nb = 0;  // red and black rows (nr = 0: the pattern has another colour count)
+  struct Half {
+    int64_t nval = 0;
+    const int32_t *sptr = nullptr, *col = nullptr;
+    const int16_t *off = nullptr;  // column minus row as 16 bits (null: too far)
+    const int32_t *src = nullptr;  // J entry of a value, -1: padding
+    const int32_t *row = nullptr;  // dof of each row of this colour
+  } e, f;                          // red rows over black columns; black rows over red columns
+  const int32_t *tsrc = nullptr;   // per f value: J entry (column, row), -1: none
+};
+
 // multicolour ILU(0) structure (permuted CSR); cptr is a host array
 struct IluStruct {
+  RedBlack rb;
   int ncolors = 0;
   std::vector<int32_t> cptr;
   const int32_t *rowptr = nullptr, *colind = nullptr, *diag = nullptr, *perm = nullptr;
@@ -160,7 +176,7 @@ class LinearSolver {
   template <class V>
   V *iluy_ptr();
   template <class V, int NDOT, int STAGE>
-  void apply_op(const V *x, V *y, const V *w0, const V *w1, KState *stp, const double *J);
+  void apply_op(const V *x, V *y, const V *w0, KState *stp, double *part);
   // stag_window > 0: stop (unconverged) once the residual has not fallen below 0.9 x its
   // best value for stag_window iterations
   template <class V, class VBin, class VXo>
@@ -170,6 +186,14 @@ class LinearSolver {
   int gmres(const VBin *b, VXo *x, const double *J, const vfvm_control_t &c, double rtol, double atol, int maxit,
             int &iters);
   void read_state(KState &h);
+  // one BiCGStab iteration's launches in the forms of vfvm_bicgstab.h
+  template <class V, class VXo>
+  struct Bicg;
+  // the two-colour form is used for this control
+  bool red_black(const vfvm_control_t &c) const {
+    return c.precon == VFVM_PRECON_ILU0 && c.krylov == VFVM_KRYLOV_BICGSTAB && L.ilu && L.ilu->rb.nr > 0;
+  }
+  void prepare_red_black(const double *J, bool fp32);
   // pinned status slots and their events for the pipelined Krylov loop
   KState *hst[2] = {nullptr, nullptr};
   hipEvent_t sev[2] = {nullptr, nullptr};
@@ -177,6 +201,9 @@ class LinearSolver {
   LinSetup L;
   hipStream_t stream = nullptr;
   DevBuf<KState> st;
+  DevBuf<double> part_alpha, part_omega, part_rho;  // partials of BiCGStab's three reductions
+  DevBuf<double> rb_e64, rb_f64, rb_d64;             // two-colour values: red, black, 1 / pivot
+  DevBuf<float> rb_e32, rb_f32, rb_d32;
   DevBuf<double> partials, rowscale, binv, bhat, rres, ilu64, iluy64, vbasis64;
   DevBuf<double> A64s, ilu64s;  // row-scaled operator / factor in SELL-64 order (FP64 Krylov)
   DevBuf<float> A32, ilu32s, iluy32, vbasis32, rhs32, d32;

@@ -127,8 +127,9 @@ __global__ void __launch_bounds__(VB) k_spmv(int64_t nrows, const int32_t *__res
 
 // SELL-64 SpMV of the row-scaled operator: y = Ahat x, one lane per row.  A wave
 // covers one slice of 64 rows, so each load of entry j (values and column indices)
-// is one coalesced access; no row pointers, no cross-lane reduction.  Fused dots as
-// in k_spmv.  Rows past nrows exist only as padding of the last slice.
+// is one coalesced access; no row pointers, no cross-lane reduction.  Fused dots
+// (w0, y), (y, y) and (w0, w0), the first NDOT of them.  Rows past nrows exist only as padding
+// of the last slice.
 // matrix stream loads; NT: non-temporal (the values and indices are read once per
 // application, so they need not displace the gathered vector from the caches)
 template <bool NT, class T>
@@ -146,7 +147,7 @@ __global__ void __launch_bounds__(VB) k_sell_spmv(int64_t nrows, const int32_t *
                                                   const VX *__restrict__ w0, double *partials, KState *st) {
   if (st && idle(st)) return;
   if (STAGE == STAGE_OMEGA && st->half) return;
-  double d0 = 0.0, d1 = 0.0;
+  double d0 = 0.0, d1 = 0.0, d2 = 0.0;
   for (int64_t r = (int64_t)blockIdx.x * VB + threadIdx.x; r < nrows; r += (int64_t)gridDim.x * VB) {
     const int64_t sl = r >> 6;
     const int32_t p1 = sptr[sl + 1];
@@ -158,10 +159,17 @@ __global__ void __launch_bounds__(VB) k_sell_spmv(int64_t nrows, const int32_t *
     y[r] = yv;
     if (NDOT >= 1) d0 += (double)w0[r] * (double)yv;
     if (NDOT >= 2) d1 += (double)yv * (double)yv;
+    if (NDOT >= 3) d2 += (double)w0[r] * (double)w0[r];
   }
-  if constexpr (NDOT > 0) {
+  if constexpr (NDOT == 1) {
+    double v[1] = {d0};
+    write_partials<1>(v, partials);
+  } else if constexpr (NDOT == 2) {
     double v[2] = {d0, d1};
     write_partials<2>(v, partials);
+  } else if constexpr (NDOT == 3) {
+    double v[3] = {d0, d1, d2};
+    write_partials<3>(v, partials);
   }
 }
 
@@ -209,57 +217,6 @@ __global__ void __launch_bounds__(VB) k_scaled_residual(int64_t nrows, const int
 }
 
 // ---------------------------------------------------------- BiCGStab -------
-// p = r + beta (p - omega v)
-template <class V>
-__global__ void __launch_bounds__(VB) k_bicg_p(int64_t n, const V *__restrict__ r, V *__restrict__ p,
-                                               const V *__restrict__ v, const KState *st) {
-  if (idle(st)) return;
-  const double beta = st->beta, omega = st->omega;
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
-    p[i] = (V)((double)r[i] + beta * ((double)p[i] - omega * (double)v[i]));
-}
-
-// s = r - alpha v ; ss = (s, s)
-template <class V>
-__global__ void __launch_bounds__(VB) k_bicg_s(int64_t n, const V *__restrict__ r, const V *__restrict__ v,
-                                               V *__restrict__ s, double *partials, KState *st) {
-  if (idle(st)) return;
-  const double alpha = st->alpha;
-  double d = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
-    const V sv = (V)((double)r[i] - alpha * (double)v[i]);
-    s[i] = sv;
-    d += (double)sv * (double)sv;
-  }
-  double vv[1] = {d};
-  write_partials<1>(vv, partials);
-}
-
-// x += alpha ph + omega sh ; r = s - omega t ; (r0, r), (r, r)
-template <class V, class VXo>
-__global__ void __launch_bounds__(VB) k_bicg_xr(int64_t n, VXo *__restrict__ x, const V *__restrict__ ph,
-                                                const V *__restrict__ sh, const V *__restrict__ s,
-                                                const V *__restrict__ t, V *__restrict__ r, const V *__restrict__ r0,
-                                                double *partials, KState *st) {
-  if (idle(st)) return;
-  const double alpha = st->alpha, omega = st->omega;
-  const bool half = st->half != 0;
-  double d0 = 0.0, d1 = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
-    if (half) {
-      x[i] = (VXo)((double)x[i] + alpha * (double)ph[i]);
-    } else {
-      x[i] = (VXo)((double)x[i] + alpha * (double)ph[i] + omega * (double)sh[i]);
-      const V rv = (V)((double)s[i] - omega * (double)t[i]);
-      r[i] = rv;
-      d0 += (double)r0[i] * (double)rv;
-      d1 += (double)rv * (double)rv;
-    }
-  }
-  double vv[2] = {d0, d1};
-  write_partials<2>(vv, partials);
-}
-
 // start: r = r0 = b (x = 0), (r, r) -> rho, rr; tolerance from ||b||
 template <class V, class VB_>
 __global__ void __launch_bounds__(VB) k_bicg_init(int64_t n, const VB_ *__restrict__ b, V *__restrict__ r,
@@ -711,6 +668,8 @@ __global__ void __launch_bounds__(VB) k_maxdiff(int64_t n, const double *__restr
   }
 }
 
+#include "vfvm_bicgstab.h"
+
 // CSC gather: out[k] = J[perm[k]]
 __global__ void __launch_bounds__(VB) k_gather(int64_t n, const int32_t *__restrict__ perm, const double *__restrict__ J,
                                                double *__restrict__ out) {
@@ -732,12 +691,15 @@ void LinearSolver::setup(const LinSetup &ls, hipStream_t s) {
   L = ls;
   stream = s;
   int64_t n = L.ndof;
-  st.alloc(1);
+  st.alloc(4);
   for (int i = 0; i < 2; i++) {
     if (!hst[i]) VFVM_HIP_CHECK(hipHostMalloc((void **)&hst[i], sizeof(KState), hipHostMallocDefault));
     if (!sev[i]) VFVM_HIP_CHECK(hipEventCreateWithFlags(&sev[i], hipEventDisableTiming));
   }
   partials.alloc((size_t)4 * MAX_RED_BLOCKS);
+  part_alpha.alloc((size_t)2 * MAX_RED_BLOCKS);
+  part_omega.alloc((size_t)6 * MAX_RED_BLOCKS);
+  part_rho.alloc((size_t)4 * MAX_RED_BLOCKS);
   rowscale.alloc((size_t)n);
   // the ILU structure may have been rebuilt in another ordering: factor copies are
   // reallocated, so that the SELL padding of the new layout starts at zero
@@ -745,8 +707,8 @@ void LinearSolver::setup(const LinSetup &ls, hipStream_t s) {
   ilu_sell_ready[0] = ilu_sell_ready[1] = false;
   ilu32s.release();
   ilu64s.release();
-  hipLaunchKernelGGL((k_fill<unsigned char>), dim3(grid_for((int64_t)sizeof(KState))), dim3(VB), 0, s,
-                     (int64_t)sizeof(KState), reinterpret_cast<unsigned char *>(st.p), (unsigned char)0);
+  hipLaunchKernelGGL((k_fill<unsigned char>), dim3(grid_for((int64_t)(4 * sizeof(KState)))), dim3(VB), 0, s,
+                     (int64_t)(4 * sizeof(KState)), reinterpret_cast<unsigned char *>(st.p), (unsigned char)0);
   hipLaunchKernelGGL((k_fill<double>), dim3(grid_for(4 * MAX_RED_BLOCKS)), dim3(VB), 0, s,
                      (int64_t)4 * MAX_RED_BLOCKS, partials.p, 0.0);
   VFVM_HIP_CHECK(hipGetLastError());
@@ -858,7 +820,8 @@ void LinearSolver::prepare(const double *J, const vfvm_control_t &c, bool refact
     ilu_ready = true;
     ilu_sell_ready[0] = ilu_sell_ready[1] = false;
   }
-  if (ilu && !ilu_sell_ready[fp32 ? 0 : 1]) {
+  if (red_black(c)) prepare_red_black(J, fp32);
+  else if (ilu && !ilu_sell_ready[fp32 ? 0 : 1]) {
     const IluStruct &I = *L.ilu;
     if (fp32) {
       if (ilu32s.n != (size_t)I.snnz) {
@@ -934,11 +897,9 @@ V *LinearSolver::iluy_ptr() {
   }
 }
 
-// y = Ahat x with optional fused dots, in the working precision V
+// y = Ahat x with optional fused dots (partials to `part`), in the working precision V
 template <class V, int NDOT, int STAGE>
-void LinearSolver::apply_op(const V *x, V *y, const V *w0, const V *w1, KState *stp, const double *J) {
-  (void)w1;
-  (void)J;
+void LinearSolver::apply_op(const V *x, V *y, const V *w0, KState *stp, double *part) {
   const unsigned g = grid_for(L.ndof);
   const int kid = sizeof(V) == 4 ? VFVM_KERNEL_SPMV32 : VFVM_KERNEL_SPMV64;
   if (L.probe) L.probe->before(kid, stream);
@@ -947,10 +908,10 @@ void LinearSolver::apply_op(const V *x, V *y, const V *w0, const V *w1, KState *
     using CI = std::remove_const_t<std::remove_pointer_t<decltype(col)>>;
     if constexpr (sizeof(V) == 4)
       VFVM_LAUNCH((k_sell_spmv<float, V, NDOT, STAGE, NT, CI>), dim3(g), dim3(VB), 0, stream, L.ndof, L.sell_ptr, col,
-                  (const float *)A32.p, x, y, w0, partials.p, stp);
+                  (const float *)A32.p, x, y, w0, part, stp);
     else
       VFVM_LAUNCH((k_sell_spmv<double, V, NDOT, STAGE, NT, CI>), dim3(g), dim3(VB), 0, stream, L.ndof, L.sell_ptr,
-                  col, (const double *)A64s.p, x, y, w0, partials.p, stp);
+                  col, (const double *)A64s.p, x, y, w0, part, stp);
   };
   const bool nt = sell_nt[sizeof(V) == 4 ? 0 : 1];
   if (L.sell_off16 && sell16) {
@@ -965,17 +926,14 @@ void LinearSolver::apply_op(const V *x, V *y, const V *w0, const V *w1, KState *
       go(std::false_type(), L.sell_col);
   }
   if (L.probe) L.probe->after(kid, stream, L.ndof, L.nnz);
-  if constexpr (NDOT > 0)
-    hipLaunchKernelGGL((k_finalize<2, STAGE>), dim3(1), dim3(VB), 0, stream, (const double *)partials.p, (int)g, stp, 1);
 }
 
 void LinearSolver::apply_plain(bool fp32, const double *J, const void *x, void *y) {
+  (void)J;
   if (fp32)
-    apply_op<float, 0, STAGE_NONE>((const float *)x, (float *)y, (const float *)nullptr, (const float *)nullptr,
-                                   nullptr, J);
+    apply_op<float, 0, STAGE_NONE>((const float *)x, (float *)y, (const float *)nullptr, nullptr, nullptr);
   else
-    apply_op<double, 0, STAGE_NONE>((const double *)x, (double *)y, (const double *)nullptr,
-                                    (const double *)nullptr, nullptr, J);
+    apply_op<double, 0, STAGE_NONE>((const double *)x, (double *)y, (const double *)nullptr, nullptr, nullptr);
   VFVM_HIP_CHECK(hipGetLastError());
 }
 
@@ -984,24 +942,215 @@ void LinearSolver::read_state(KState &h) {
   VFVM_HIP_CHECK(hipStreamSynchronize(stream));
 }
 
+// values of the two-colour form from J and the row scaling, in the solve precision
+void LinearSolver::prepare_red_black(const double *J, bool fp32) {
+  const RedBlack &R = L.ilu->rb;
+  auto go = [&](auto &e, auto &f, auto &d) {
+    using V = std::remove_reference_t<decltype(*e.p)>;
+    e.alloc((size_t)R.e.nval);
+    f.alloc((size_t)R.f.nval);
+    d.alloc((size_t)R.nb);
+    hipLaunchKernelGGL((k_rb_values<V, false>), dim3((unsigned)((R.nr + VB - 1) / VB)), dim3(VB), 0, stream, R.nr,
+                       R.e.sptr, R.e.src, (const int32_t *)nullptr, R.e.row, L.colind, L.dofdiag, J,
+                       (const double *)rowscale.p, e.p, (V *)nullptr);
+    hipLaunchKernelGGL((k_rb_values<V, true>), dim3((unsigned)((R.nb + VB - 1) / VB)), dim3(VB), 0, stream, R.nb,
+                       R.f.sptr, R.f.src, R.tsrc, R.f.row, L.colind, L.dofdiag, J, (const double *)rowscale.p, f.p,
+                       d.p);
+  };
+  if (fp32)
+    go(rb_e32, rb_f32, rb_d32);
+  else
+    go(rb_e64, rb_f64, rb_d64);
+  VFVM_HIP_CHECK(hipGetLastError());
+}
+
+// rows up to which the point Jacobi form also forms the search direction inside the product
+// (three gathered vectors instead of one, but one launch less).  An iteration took, fused and
+// not, 16.2 and 20.0 us at 33^2 rows, 17.9 and 19.6 us at 257^2 (also 33^3: 17.9 and 20.1), and
+// the same from 363^2 on (23.9 and 24.2; 51^3: 29.1 and 29.6; 513^2: 31.9 and 31.8).
+constexpr int64_t FUSE_P_ROWS = 1 << 17;
+
+// The launches of BiCGStab in the form that fits the preconditioner.  init() sets the start
+// state (slot 0 and the partials of (r, r)), iterate(first) queues one iteration, report() the
+// host's copy of the state after it (slot 3).
+template <class V, class VXo>
+struct LinearSolver::Bicg {
+  LinearSolver &S;
+  const vfvm_control_t &c;
+  VXo *x;
+  hipStream_t st;
+  int64_t n;
+  unsigned g;
+  V *r, *r0, *p, *v, *s, *t, *ph, *sh, *xx;
+  KState *k;
+  const bool rb, blk, plain;
+  int nrho = 0;  // partials of the last (r0, r), (r, r)
+  Bicg(LinearSolver &ls, const vfvm_control_t &cc, VXo *xo)
+      : S(ls), c(cc), x(xo), st(ls.stream), n(ls.L.ndof), g(grid_for(ls.L.ndof)), k(ls.st.p), rb(ls.red_black(cc)),
+        blk(cc.precon == VFVM_PRECON_BLOCKJACOBI && ls.L.nspec > 1),
+        plain(cc.precon == VFVM_PRECON_JACOBI || (cc.precon == VFVM_PRECON_BLOCKJACOBI && ls.L.nspec == 1)) {
+    Work<V> &W = S.work<V>();
+    r = W.vecs[0].p, r0 = W.vecs[1].p, p = W.vecs[2].p, v = W.vecs[3].p, s = W.vecs[4].p, t = W.vecs[5].p,
+    ph = W.vecs[6].p, sh = W.vecs[7].p, xx = W.vecs[8].p;
+  }
+  // matrix values, column indices and their load form of the SELL-64 operator
+  template <class F>
+  void with_operator(F &&f) {
+    const V *val;
+    if constexpr (sizeof(V) == 4) val = S.A32.p;
+    else val = S.A64s.p;
+    const bool nt = S.sell_nt[sizeof(V) == 4 ? 0 : 1];
+    if (S.L.sell_off16 && S.sell16) {
+      if (nt) f(std::true_type(), S.L.sell_off16, val);
+      else f(std::false_type(), S.L.sell_off16, val);
+    } else {
+      if (nt) f(std::true_type(), S.L.sell_col, val);
+      else f(std::false_type(), S.L.sell_col, val);
+    }
+  }
+  template <class VBin>
+  void init(const VBin *b) {
+    if (rb) {
+      const RedBlack &R = S.L.ilu->rb;
+      hipLaunchKernelGGL((k_rb_init<V, VBin>), dim3(g), dim3(VB), 0, st, R.nr, n, R.e.row, R.f.row, b, r, r0, p, v, xx,
+                         S.part_rho.p);
+    } else {
+      hipLaunchKernelGGL((k_fill<VXo>), dim3(g), dim3(VB), 0, st, n, x, (VXo)0);
+      hipLaunchKernelGGL((k_bicg_init<V, VBin>), dim3(g), dim3(VB), 0, st, n, b, r, r0, p, v, S.part_rho.p, k);
+    }
+    nrho = (int)g;
+  }
+  void iterate(bool first) {
+    if (first)
+      iterate_at(std::integral_constant<int, STAGE_INIT>());
+    else
+      iterate_at(std::integral_constant<int, STAGE_XR>());
+  }
+  template <class ST>
+  void iterate_at(ST) {
+    constexpr int STAGE = ST::value;
+    KState *k0 = k + SLOT_RHO, *k1 = k + SLOT_BETA, *k2 = k + SLOT_ALPHA;
+    const double *rho = S.part_rho.p, *al = S.part_alpha.p, *om = S.part_omega.p;
+    const int kid = sizeof(V) == 4 ? VFVM_KERNEL_SPMV32 : VFVM_KERNEL_SPMV64;
+    if (rb) {
+      if (S.L.ilu->rb.e.off && S.L.ilu->rb.f.off)
+        iterate_rb<STAGE, true>();
+      else
+        iterate_rb<STAGE, false>();
+    } else if (plain) {
+      const bool fuse = n <= FUSE_P_ROWS;
+      with_operator([&](auto ntc, const auto *col, const V *val) {
+        constexpr bool NT = decltype(ntc)::value;
+        using CI = std::remove_const_t<std::remove_pointer_t<decltype(col)>>;
+        if (fuse) {
+          hipLaunchKernelGGL((k_bicg_pv<V, STAGE, NT, CI>), dim3(g), dim3(VB), 0, st, n, S.L.sell_ptr, col, val, r, p,
+                             v, ph, s, r0, rho, nrho, k0, k1, S.part_alpha.p);
+          std::swap(p, ph);
+          std::swap(v, s);
+        } else {
+          hipLaunchKernelGGL((k_bicg_p<V, STAGE, 0>), dim3(g), dim3(VB), 0, st, n, r, p, v, (const double *)nullptr,
+                             (V *)nullptr, rho, nrho, k0, k1);
+          S.apply_op<V, 1, STAGE_NONE>(p, v, r0, k1, S.part_alpha.p);
+        }
+        if (S.L.probe) S.L.probe->before(kid, st);
+        VFVM_LAUNCH((k_bicg_st<V, NT, CI>), dim3(g), dim3(VB), 0, st, n, S.L.sell_ptr, col, val, r, v, t, al, (int)g,
+                    k1, k2, S.part_omega.p);
+        if (S.L.probe) S.L.probe->after(kid, st, S.L.ndof, S.L.nnz);
+      });
+      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_SOMEGA, true>), dim3(g), dim3(VB), 0, st, n, x, p, (const V *)nullptr,
+                         (const V *)nullptr, v, t, r, r0, om, (int)g, k2, k0, S.part_rho.p);
+    } else if (blk) {
+      auto go = [&](auto ns) {
+        constexpr int NS = decltype(ns)::value;
+        const unsigned gn = grid_for(S.L.nnodes);
+        hipLaunchKernelGGL((k_bicg_p<V, STAGE, NS>), dim3(gn), dim3(VB), 0, st, S.L.nnodes, r, p, v,
+                           (const double *)S.binv.p, ph, rho, nrho, k0, k1);
+        S.apply_op<V, 1, STAGE_NONE>(ph, v, r0, k1, S.part_alpha.p);
+        hipLaunchKernelGGL((k_bicg_s<V, NS, false>), dim3(gn), dim3(VB), 0, st, S.L.nnodes, r, v, s,
+                           (const double *)S.binv.p, sh, al, (int)g, k1, k2, (double *)nullptr);
+      };
+      if (S.L.nspec == 2) go(std::integral_constant<int, 2>());
+      else go(std::integral_constant<int, 3>());
+      S.apply_op<V, 3, STAGE_NONE>(sh, t, s, k2, S.part_omega.p);
+      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_SOMEGA, false>), dim3(g), dim3(VB), 0, st, n, x, ph, sh, s, v, t, r,
+                         r0, om, (int)g, k2, k0, S.part_rho.p);
+    } else {
+      // a costly preconditioner: its second application and product are skipped when the half
+      // step has converged, which takes a launch to decide
+      hipLaunchKernelGGL((k_bicg_p<V, STAGE, 0>), dim3(g), dim3(VB), 0, st, n, r, p, v, (const double *)nullptr,
+                         (V *)nullptr, rho, nrho, k0, k1);
+      const V *php = S.precond<V>(p, ph, k1, 0, c);
+      S.apply_op<V, 1, STAGE_NONE>(php, v, r0, k1, S.part_alpha.p);
+      hipLaunchKernelGGL((k_bicg_s<V, 0, true>), dim3(g), dim3(VB), 0, st, n, r, v, s, (const double *)nullptr,
+                         (V *)nullptr, al, (int)g, k1, k2, S.partials.p);
+      hipLaunchKernelGGL((k_finalize<1, STAGE_SNORM>), dim3(1), dim3(VB), 0, st, (const double *)S.partials.p, (int)g,
+                         k2, 1);
+      const V *shp = S.precond<V>(s, sh, k2, 1, c);
+      S.apply_op<V, 2, STAGE_OMEGA>(shp, t, s, k2, S.part_omega.p);
+      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_OMEGA, false>), dim3(g), dim3(VB), 0, st, n, x, php, shp, s, v, t, r,
+                         r0, om, (int)g, k2, k0, S.part_rho.p);
+    }
+    nrho = (int)g;
+  }
+  template <int STAGE, bool OFF>
+  void iterate_rb() {
+    const RedBlack &R = S.L.ilu->rb;
+    RbMat<V> A;
+    A.nr = R.nr;
+    A.nb = R.nb;
+    A.es = R.e.sptr;
+    A.fs = R.f.sptr;
+    A.eo = R.e.off;
+    A.fo = R.f.off;
+    A.ec = R.e.col;
+    A.fc = R.f.col;
+    if constexpr (sizeof(V) == 4) {
+      A.ev = S.rb_e32.p;
+      A.fv = S.rb_f32.p;
+      A.d = S.rb_d32.p;
+    } else {
+      A.ev = S.rb_e64.p;
+      A.fv = S.rb_f64.p;
+      A.d = S.rb_d64.p;
+    }
+    KState *k0 = k + SLOT_RHO, *k1 = k + SLOT_BETA, *k2 = k + SLOT_ALPHA;
+    const unsigned gr = grid_for(R.nr), gb = grid_for(R.nb);
+    const int np = (int)(gr + gb);
+    double *al = S.part_alpha.p, *om = S.part_omega.p;
+    hipLaunchKernelGGL((k_rb_p_black<V, STAGE, OFF>), dim3(gb), dim3(VB), 0, st, A, r, p, v, ph,
+                       (const double *)S.part_rho.p, nrho, k0, k1);
+    hipLaunchKernelGGL((k_rb_p_red<V, OFF>), dim3(gr), dim3(VB), 0, st, A, r, p, ph, r0, k1, al, np);
+    hipLaunchKernelGGL((k_rb_v<V, OFF>), dim3(gb), dim3(VB), 0, st, A, ph, v, r0, k1, al, np, (int)gr);
+    hipLaunchKernelGGL((k_rb_s_black<V, OFF>), dim3(gb), dim3(VB), 0, st, A, r, p, v, sh, (const double *)al, np, k1,
+                       k2);
+    hipLaunchKernelGGL((k_rb_s_red<V, OFF>), dim3(gr), dim3(VB), 0, st, A, r, p, sh, k2, om, np);
+    hipLaunchKernelGGL((k_rb_t<V, OFF>), dim3(gb), dim3(VB), 0, st, A, r, v, sh, t, k2, om, np, (int)gr);
+    hipLaunchKernelGGL((k_rb_xr<V>), dim3(g), dim3(VB), 0, st, R.nr, n, xx, ph, sh, p, v, t, r, r0, (const double *)om,
+                       np, k2, k0, S.part_rho.p);
+  }
+  void report() {
+    hipLaunchKernelGGL(k_bicg_report, dim3(1), dim3(VB), 0, st, (const double *)S.part_rho.p, nrho, k + SLOT_RHO,
+                       k + SLOT_REPORT);
+  }
+  void finish() {
+    if (!rb) return;
+    const RedBlack &R = S.L.ilu->rb;
+    hipLaunchKernelGGL((k_rb_out<V, VXo>), dim3(g), dim3(VB), 0, st, R.nr, n, R.e.row, R.f.row, xx, x);
+  }
+};
+
 // BiCGStab on Ahat x = bhat in precision V; b is given in precision VB_ (already scaled)
 template <class V, class VBin, class VXo>
 int LinearSolver::bicgstab(const VBin *b, VXo *x, const double *J, const vfvm_control_t &c, double rtol, double atol,
                            int maxit, int &iters, int stag_window) {
-  int64_t n = L.ndof;
-  Work<V> &W = work<V>();
-  V *r = W.vecs[0].p, *r0 = W.vecs[1].p, *p = W.vecs[2].p, *v = W.vecs[3].p, *s = W.vecs[4].p, *t = W.vecs[5].p,
-    *ph = W.vecs[6].p, *sh = W.vecs[7].p;
+  (void)J;
   KState h{};
   h.maxit = maxit;
   h.rtol = rtol;
   h.atol = atol;
   VFVM_HIP_CHECK(hipMemcpyAsync(st.p, &h, sizeof(KState), hipMemcpyHostToDevice, stream));
-  unsigned g = grid_for(n);
-  hipLaunchKernelGGL((k_fill<VXo>), dim3(g), dim3(VB), 0, stream, n, x, (VXo)0);
-  hipLaunchKernelGGL((k_bicg_init<V, VBin>), dim3(g), dim3(VB), 0, stream, n, b, r, r0, p, v, partials.p, st.p);
-  hipLaunchKernelGGL((k_finalize<1, STAGE_INIT>), dim3(1), dim3(VB), 0, stream, (const double *)partials.p, (int)g, st.p,
-                     0);
+  Bicg<V, VXo> K(*this, c, x);
+  K.init(b);
   // first chunk: about as many iterations as the previous solve needed (Newton steps of one
   // solve need similar counts), then poll every check_every iterations
   const int every = std::max(1, c.check_every);
@@ -1012,23 +1161,11 @@ int LinearSolver::bicgstab(const VBin *b, VXo *x, const double *J, const vfvm_co
   // block is examined (a block queued after convergence runs kernels that return at
   // entry); each block ends with an asynchronous copy of the state into its pinned slot.
   auto enqueue = [&](int nit, int slot) {
-    for (int q = 0; q < nit; q++) {
-      hipLaunchKernelGGL((k_bicg_p<V>), dim3(g), dim3(VB), 0, stream, n, r, p, v, st.p);
-      const V *php = precond<V>(p, ph, st.p, 0, c);
-      apply_op<V, 1, STAGE_ALPHA>(php, v, r0, (const V *)nullptr, st.p, J);
-      hipLaunchKernelGGL((k_bicg_s<V>), dim3(g), dim3(VB), 0, stream, n, r, v, s, partials.p, st.p);
-      hipLaunchKernelGGL((k_finalize<1, STAGE_SNORM>), dim3(1), dim3(VB), 0, stream, (const double *)partials.p, (int)g,
-                         st.p, 1);
-      const V *shp = precond<V>(s, sh, st.p, 1, c);
-      apply_op<V, 2, STAGE_OMEGA>(shp, t, s, (const V *)nullptr, st.p, J);
-      hipLaunchKernelGGL((k_bicg_xr<V, VXo>), dim3(g), dim3(VB), 0, stream, n, x, php, shp, s, t, r, r0, partials.p,
-                         st.p);
-      hipLaunchKernelGGL((k_finalize<2, STAGE_XR>), dim3(1), dim3(VB), 0, stream, (const double *)partials.p, (int)g,
-                         st.p, 1);
-    }
+    for (int q = 0; q < nit; q++) K.iterate(launched + q == 0);
+    K.report();
     VFVM_HIP_CHECK(hipGetLastError());
     launched += nit;
-    VFVM_HIP_CHECK(hipMemcpyAsync(hst[slot], st.p, sizeof(KState), hipMemcpyDeviceToHost, stream));
+    VFVM_HIP_CHECK(hipMemcpyAsync(hst[slot], st.p + SLOT_REPORT, sizeof(KState), hipMemcpyDeviceToHost, stream));
     VFVM_HIP_CHECK(hipEventRecord(sev[slot], stream));
   };
   int slot = 0, last = 0;
@@ -1054,6 +1191,8 @@ int LinearSolver::bicgstab(const VBin *b, VXo *x, const double *J, const vfvm_co
   }
   VFVM_HIP_CHECK(hipEventSynchronize(sev[last]));  // state after the last queued block
   h = *hst[last];
+  K.finish();
+  VFVM_HIP_CHECK(hipGetLastError());
   iters = h.iters;
   last_iters = h.iters;
   last_rr = h.rr;
@@ -1113,7 +1252,7 @@ int LinearSolver::gmres(const VBin *b, VXo *x, const double *J, const vfvm_contr
     for (; k < m; k++) {
       V *vk = Vb + (int64_t)k * n, *vk1 = Vb + (int64_t)(k + 1) * n;
       const V *zp = precond<V>(vk, z, nullptr, 0, c);
-      apply_op<V, 0, STAGE_NONE>(zp, w, (const V *)nullptr, (const V *)nullptr, nullptr, J);
+      apply_op<V, 0, STAGE_NONE>(zp, w, (const V *)nullptr, nullptr, nullptr);
       // CGS2: two passes of (h = V^T w ; w -= V h)
       for (int pass = 0; pass < 2; pass++) {
         double *hh = pass == 0 ? gmh1.p : gmh2.p;

@@ -45,6 +45,12 @@ struct vfvm_sys {
   bool has_gen = false;
   DevBuf<int32_t> d_ilu_rowptr, d_ilu_colind, d_ilu_diag, d_ilu_perm, d_ilu_src, d_ilu_srcrow, d_ilu_sptr,
       d_ilu_scol, d_ilu_sdpos;
+  // its two-colour form
+  struct RbHalf {
+    DevBuf<int32_t> sptr, col, src, row;
+    DevBuf<int16_t> off;
+  } d_rb_e, d_rb_f;
+  DevBuf<int32_t> d_rb_tsrc;
   // SELL-64 copy of the Jacobian pattern for the Krylov operator
   DevBuf<int32_t> d_sell_ptr, d_sell_col, d_sell_rbase;
   DevBuf<int16_t> d_sell_off16;  // empty when some row reaches further than 32767 rows
