@@ -30,10 +30,30 @@ namespace {
 
 constexpr int VB = 256;  // threads per block of vector kernels
 
+// v plus the v of the lane that the DPP control CTRL selects in its row of 16
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return v + __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true),
+                              __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// sum over the wave (all 64 lanes active), the same value in every lane.  The steps within a row
+// of 16 lanes are register moves (a butterfly through LDS takes about 100 cycles per step).
+__device__ __forceinline__ double wave_sum(double v) {
+  v = add_dpp<0xB1>(v);   // lane ^ 1
+  v = add_dpp<0x4E>(v);   // lane ^ 2
+  v = add_dpp<0x141>(v);  // mirrored within 8 lanes
+  v = add_dpp<0x140>(v);  // mirrored within 16 lanes
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
 __device__ __forceinline__ double block_sum(double v, double *sh) {
   // wave reduction then across the 4 waves of the block
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_sum(v);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   __syncthreads();
   if (l == 0) sh[w] = v;
@@ -687,6 +707,15 @@ static unsigned grid_for(int64_t n, int per_thread_rows = 1) {
   return (unsigned)b;
 }
 
+// Blocks of the vector updates of BiCGStab.  Each of them sums all partials of the product
+// before it, and its own partials are summed by every block of the product after it, so fewer
+// blocks than a pure stream wants: on 129^3 rows in FP32 the update of x and r takes 21.9 us
+// with 2048 blocks, 16.7 with 1024 and 16.1 with 512, and the product after it 20.5, 19.6 and
+// 18.6.  The products keep one row per thread as far as it goes (13.4 us with 1024 blocks and
+// 18.1 with 512, against 11.5).
+constexpr unsigned FOLD_BLOCKS = 512;
+static unsigned fold_blocks(int64_t n) { return std::min(grid_for(n), FOLD_BLOCKS); }
+
 void LinearSolver::setup(const LinSetup &ls, hipStream_t s) {
   L = ls;
   stream = s;
@@ -972,7 +1001,7 @@ constexpr int64_t FUSE_P_ROWS = 1 << 17;
 
 // The launches of BiCGStab in the form that fits the preconditioner.  init() sets the start
 // state (slot 0 and the partials of (r, r)), iterate(first) queues one iteration, report() the
-// host's copy of the state after it (slot 3).
+// host's copy of the state after it.
 template <class V, class VXo>
 struct LinearSolver::Bicg {
   LinearSolver &S;
@@ -980,13 +1009,13 @@ struct LinearSolver::Bicg {
   VXo *x;
   hipStream_t st;
   int64_t n;
-  unsigned g;
+  unsigned g, gv;  // blocks of the products, of the vector updates
   V *r, *r0, *p, *v, *s, *t, *ph, *sh, *xx;
   KState *k;
   const bool rb, blk, plain;
   int nrho = 0;  // partials of the last (r0, r), (r, r)
   Bicg(LinearSolver &ls, const vfvm_control_t &cc, VXo *xo)
-      : S(ls), c(cc), x(xo), st(ls.stream), n(ls.L.ndof), g(grid_for(ls.L.ndof)), k(ls.st.p), rb(ls.red_black(cc)),
+      : S(ls), c(cc), x(xo), st(ls.stream), n(ls.L.ndof), g(grid_for(ls.L.ndof)), gv(fold_blocks(ls.L.ndof)), k(ls.st.p), rb(ls.red_black(cc)),
         blk(cc.precon == VFVM_PRECON_BLOCKJACOBI && ls.L.nspec > 1),
         plain(cc.precon == VFVM_PRECON_JACOBI || (cc.precon == VFVM_PRECON_BLOCKJACOBI && ls.L.nspec == 1)) {
     Work<V> &W = S.work<V>();
@@ -1012,13 +1041,13 @@ struct LinearSolver::Bicg {
   void init(const VBin *b) {
     if (rb) {
       const RedBlack &R = S.L.ilu->rb;
-      hipLaunchKernelGGL((k_rb_init<V, VBin>), dim3(g), dim3(VB), 0, st, R.nr, n, R.e.row, R.f.row, b, r, r0, p, v, xx,
+      hipLaunchKernelGGL((k_rb_init<V, VBin>), dim3(gv), dim3(VB), 0, st, R.nr, n, R.e.row, R.f.row, b, r, r0, p, v, xx,
                          S.part_rho.p);
     } else {
       hipLaunchKernelGGL((k_fill<VXo>), dim3(g), dim3(VB), 0, st, n, x, (VXo)0);
-      hipLaunchKernelGGL((k_bicg_init<V, VBin>), dim3(g), dim3(VB), 0, st, n, b, r, r0, p, v, S.part_rho.p, k);
+      hipLaunchKernelGGL((k_bicg_init<V, VBin>), dim3(gv), dim3(VB), 0, st, n, b, r, r0, p, v, S.part_rho.p, k);
     }
-    nrho = (int)g;
+    nrho = (int)gv;
   }
   void iterate(bool first) {
     if (first)
@@ -1033,10 +1062,11 @@ struct LinearSolver::Bicg {
     const double *rho = S.part_rho.p, *al = S.part_alpha.p, *om = S.part_omega.p;
     const int kid = sizeof(V) == 4 ? VFVM_KERNEL_SPMV32 : VFVM_KERNEL_SPMV64;
     if (rb) {
-      if (S.L.ilu->rb.e.off && S.L.ilu->rb.f.off)
-        iterate_rb<STAGE, true>();
+      const RedBlack &R = S.L.ilu->rb;
+      if (R.e.off && R.f.off)
+        iterate_rb<STAGE, int16_t>(R.e.off, R.f.off);
       else
-        iterate_rb<STAGE, false>();
+        iterate_rb<STAGE, int32_t>(R.e.col, R.f.col);
     } else if (plain) {
       const bool fuse = n <= FUSE_P_ROWS;
       with_operator([&](auto ntc, const auto *col, const V *val) {
@@ -1048,7 +1078,7 @@ struct LinearSolver::Bicg {
           std::swap(p, ph);
           std::swap(v, s);
         } else {
-          hipLaunchKernelGGL((k_bicg_p<V, STAGE, 0>), dim3(g), dim3(VB), 0, st, n, r, p, v, (const double *)nullptr,
+          hipLaunchKernelGGL((k_bicg_p<V, STAGE, 0>), dim3(gv), dim3(VB), 0, st, n, r, p, v, (const double *)nullptr,
                              (V *)nullptr, rho, nrho, k0, k1);
           S.apply_op<V, 1, STAGE_NONE>(p, v, r0, k1, S.part_alpha.p);
         }
@@ -1057,12 +1087,12 @@ struct LinearSolver::Bicg {
                     k1, k2, S.part_omega.p);
         if (S.L.probe) S.L.probe->after(kid, st, S.L.ndof, S.L.nnz);
       });
-      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_SOMEGA, true>), dim3(g), dim3(VB), 0, st, n, x, p, (const V *)nullptr,
+      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_SOMEGA, true>), dim3(gv), dim3(VB), 0, st, n, x, p, (const V *)nullptr,
                          (const V *)nullptr, v, t, r, r0, om, (int)g, k2, k0, S.part_rho.p);
     } else if (blk) {
       auto go = [&](auto ns) {
         constexpr int NS = decltype(ns)::value;
-        const unsigned gn = grid_for(S.L.nnodes);
+        const unsigned gn = fold_blocks(S.L.nnodes);
         hipLaunchKernelGGL((k_bicg_p<V, STAGE, NS>), dim3(gn), dim3(VB), 0, st, S.L.nnodes, r, p, v,
                            (const double *)S.binv.p, ph, rho, nrho, k0, k1);
         S.apply_op<V, 1, STAGE_NONE>(ph, v, r0, k1, S.part_alpha.p);
@@ -1072,38 +1102,36 @@ struct LinearSolver::Bicg {
       if (S.L.nspec == 2) go(std::integral_constant<int, 2>());
       else go(std::integral_constant<int, 3>());
       S.apply_op<V, 3, STAGE_NONE>(sh, t, s, k2, S.part_omega.p);
-      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_SOMEGA, false>), dim3(g), dim3(VB), 0, st, n, x, ph, sh, s, v, t, r,
+      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_SOMEGA, false>), dim3(gv), dim3(VB), 0, st, n, x, ph, sh, s, v, t, r,
                          r0, om, (int)g, k2, k0, S.part_rho.p);
     } else {
       // a costly preconditioner: its second application and product are skipped when the half
       // step has converged, which takes a launch to decide
-      hipLaunchKernelGGL((k_bicg_p<V, STAGE, 0>), dim3(g), dim3(VB), 0, st, n, r, p, v, (const double *)nullptr,
+      hipLaunchKernelGGL((k_bicg_p<V, STAGE, 0>), dim3(gv), dim3(VB), 0, st, n, r, p, v, (const double *)nullptr,
                          (V *)nullptr, rho, nrho, k0, k1);
       const V *php = S.precond<V>(p, ph, k1, 0, c);
       S.apply_op<V, 1, STAGE_NONE>(php, v, r0, k1, S.part_alpha.p);
-      hipLaunchKernelGGL((k_bicg_s<V, 0, true>), dim3(g), dim3(VB), 0, st, n, r, v, s, (const double *)nullptr,
+      hipLaunchKernelGGL((k_bicg_s<V, 0, true>), dim3(gv), dim3(VB), 0, st, n, r, v, s, (const double *)nullptr,
                          (V *)nullptr, al, (int)g, k1, k2, S.partials.p);
-      hipLaunchKernelGGL((k_finalize<1, STAGE_SNORM>), dim3(1), dim3(VB), 0, st, (const double *)S.partials.p, (int)g,
+      hipLaunchKernelGGL((k_finalize<1, STAGE_SNORM>), dim3(1), dim3(VB), 0, st, (const double *)S.partials.p, (int)gv,
                          k2, 1);
       const V *shp = S.precond<V>(s, sh, k2, 1, c);
       S.apply_op<V, 2, STAGE_OMEGA>(shp, t, s, k2, S.part_omega.p);
-      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_OMEGA, false>), dim3(g), dim3(VB), 0, st, n, x, php, shp, s, v, t, r,
+      hipLaunchKernelGGL((k_bicg_xr<V, VXo, STAGE_OMEGA, false>), dim3(gv), dim3(VB), 0, st, n, x, php, shp, s, v, t, r,
                          r0, om, (int)g, k2, k0, S.part_rho.p);
     }
-    nrho = (int)g;
+    nrho = (int)gv;
   }
-  template <int STAGE, bool OFF>
-  void iterate_rb() {
+  template <int STAGE, class CI>
+  void iterate_rb(const CI *ec, const CI *fc) {
     const RedBlack &R = S.L.ilu->rb;
-    RbMat<V> A;
+    RbMat<V, CI> A;
     A.nr = R.nr;
     A.nb = R.nb;
     A.es = R.e.sptr;
     A.fs = R.f.sptr;
-    A.eo = R.e.off;
-    A.fo = R.f.off;
-    A.ec = R.e.col;
-    A.fc = R.f.col;
+    A.ec = ec;
+    A.fc = fc;
     if constexpr (sizeof(V) == 4) {
       A.ev = S.rb_e32.p;
       A.fv = S.rb_f32.p;
@@ -1117,20 +1145,20 @@ struct LinearSolver::Bicg {
     const unsigned gr = grid_for(R.nr), gb = grid_for(R.nb);
     const int np = (int)(gr + gb);
     double *al = S.part_alpha.p, *om = S.part_omega.p;
-    hipLaunchKernelGGL((k_rb_p_black<V, STAGE, OFF>), dim3(gb), dim3(VB), 0, st, A, r, p, v, ph,
+    hipLaunchKernelGGL((k_rb_p_black<V, STAGE, CI>), dim3(gb), dim3(VB), 0, st, A, r, p, v, ph,
                        (const double *)S.part_rho.p, nrho, k0, k1);
-    hipLaunchKernelGGL((k_rb_p_red<V, OFF>), dim3(gr), dim3(VB), 0, st, A, r, p, ph, r0, k1, al, np);
-    hipLaunchKernelGGL((k_rb_v<V, OFF>), dim3(gb), dim3(VB), 0, st, A, ph, v, r0, k1, al, np, (int)gr);
-    hipLaunchKernelGGL((k_rb_s_black<V, OFF>), dim3(gb), dim3(VB), 0, st, A, r, p, v, sh, (const double *)al, np, k1,
+    hipLaunchKernelGGL((k_rb_p_red<V, CI>), dim3(gr), dim3(VB), 0, st, A, r, p, ph, r0, k1, al, np);
+    hipLaunchKernelGGL((k_rb_v<V, CI>), dim3(gb), dim3(VB), 0, st, A, ph, v, r0, k1, al, np, (int)gr);
+    hipLaunchKernelGGL((k_rb_s_black<V, CI>), dim3(gb), dim3(VB), 0, st, A, r, p, v, sh, (const double *)al, np, k1,
                        k2);
-    hipLaunchKernelGGL((k_rb_s_red<V, OFF>), dim3(gr), dim3(VB), 0, st, A, r, p, sh, k2, om, np);
-    hipLaunchKernelGGL((k_rb_t<V, OFF>), dim3(gb), dim3(VB), 0, st, A, r, v, sh, t, k2, om, np, (int)gr);
-    hipLaunchKernelGGL((k_rb_xr<V>), dim3(g), dim3(VB), 0, st, R.nr, n, xx, ph, sh, p, v, t, r, r0, (const double *)om,
+    hipLaunchKernelGGL((k_rb_s_red<V, CI>), dim3(gr), dim3(VB), 0, st, A, r, p, sh, k2, om, np);
+    hipLaunchKernelGGL((k_rb_t<V, CI>), dim3(gb), dim3(VB), 0, st, A, r, v, sh, t, k2, om, np, (int)gr);
+    hipLaunchKernelGGL((k_rb_xr<V>), dim3(gv), dim3(VB), 0, st, R.nr, n, xx, ph, sh, p, v, t, r, r0, (const double *)om,
                        np, k2, k0, S.part_rho.p);
   }
-  void report() {
+  void report(KState *pinned) {
     hipLaunchKernelGGL(k_bicg_report, dim3(1), dim3(VB), 0, st, (const double *)S.part_rho.p, nrho, k + SLOT_RHO,
-                       k + SLOT_REPORT);
+                       pinned);
   }
   void finish() {
     if (!rb) return;
@@ -1159,13 +1187,12 @@ int LinearSolver::bicgstab(const VBin *b, VXo *x, const double *J, const vfvm_co
   double best = -1.0;
   // Pipelined: the next block of iterations is queued before the state after the current
   // block is examined (a block queued after convergence runs kernels that return at
-  // entry); each block ends with an asynchronous copy of the state into its pinned slot.
+  // entry); each block ends with the state's report to its pinned slot.
   auto enqueue = [&](int nit, int slot) {
     for (int q = 0; q < nit; q++) K.iterate(launched + q == 0);
-    K.report();
+    K.report(hst[slot]);
     VFVM_HIP_CHECK(hipGetLastError());
     launched += nit;
-    VFVM_HIP_CHECK(hipMemcpyAsync(hst[slot], st.p + SLOT_REPORT, sizeof(KState), hipMemcpyDeviceToHost, stream));
     VFVM_HIP_CHECK(hipEventRecord(sev[slot], stream));
   };
   int slot = 0, last = 0;
