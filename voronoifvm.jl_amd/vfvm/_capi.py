@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import sys
 
 import numpy as np
 
@@ -241,7 +242,9 @@ class Context:
         self.handle = h
 
     def __del__(self):
-        if getattr(self, "handle", None) and _LIB is not None:
+        # At interpreter exit finalizers of objects in reference cycles run in any order, and the
+        # systems' still use the context's stream: the process's end releases it then.
+        if getattr(self, "handle", None) and _LIB is not None and not sys.is_finalizing():
             _LIB.vfvm_ctx_destroy(self.handle)
             self.handle = None
 
