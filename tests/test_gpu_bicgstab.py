@@ -1,4 +1,4 @@
-"""The forms of the single-system BiCGStab (fused point Jacobi, block Jacobi, two-colour and general ILU(0), with the
+"""The forms of the single-system BiCGStab (fused point Jacobi, block Jacobi, two-colour and general ILU(0)) and GMRES, with the
 sizes at which each changes): the row-scaled residual of the returned solution against the Jacobian on the host."""
 import numpy as np
 import pytest
@@ -33,6 +33,22 @@ def _system(name):
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_solution_meets_the_tolerance(name, precon, precision):
     print("bicgstab", name, precon, precision, flush=True)
+    _check(name, precon, precision, krylov="bicgstab")
+
+
+@pytest.mark.parametrize("name", ["grid:2", "grid:65", "grid:127:129", "grid:181:181", "grid:181:182", "exchange:17:9",
+                                  "dd2d:9"])
+@pytest.mark.parametrize("precon", ["jacobi", "blockjacobi", "ilu0"])
+@pytest.mark.parametrize("precision,restart", [("fp64", 1), ("fp64", 7), ("fp64", 64), ("fp32", 30)])
+def test_gmres_meets_the_tolerance(name, precon, precision, restart):
+    """restarts after 1, 7, 30 and 64 columns; 128 blocks and more are the two ways of summing the dot products"""
+    print("gmres", name, precon, precision, restart, flush=True)
+    if restart == 1 and name.startswith("dd2d"):
+        restart = 2
+    _check(name, precon, precision, krylov="gmres", gmres_restart=restart)
+
+
+def _check(name, precon, precision, **kw):
     sys, tstep = _system(name)
     if name.startswith("dd2d") and precon == "ilu0":
         precon = "ilu0_natural"  # the multicolour factor of this system is no preconditioner
@@ -44,7 +60,7 @@ def test_solution_meets_the_tolerance(name, precon, precision):
     A = A.tocsr()
     s = 1.0 / A.diagonal()
     b = b / np.abs(s)  # comparable rows, also where a Dirichlet penalty stands
-    kw = dict(precon=precon, precision=precision, reltol_linear=RTOL, abstol_linear=0.0, maxiters_linear=2000)
+    kw.update(precon=precon, precision=precision, reltol_linear=RTOL, abstol_linear=0.0, maxiters_linear=2000)
     for _ in range(2):  # the second call starts from the first one's iteration count
         x, st = vfvm.linsolve(sys, b, **kw)
         x = vfvm.dofs(x)

@@ -18,8 +18,6 @@ constexpr int MAX_RED_BLOCKS = 2048;
 struct KState {
   double rho, rho_old, alpha, omega, beta;
   double rr, rr0, ss, tol2, rtol, atol;
-  double dots[4];
-  double gm_inv, gm_beta;
   int32_t iters, maxit, done, status, half, gm_k, gm_conv, gm_stop;
   unsigned ticket;
   unsigned pad;
@@ -207,7 +205,7 @@ class LinearSolver {
   DevBuf<double> partials, rowscale, binv, bhat, rres, ilu64, iluy64, vbasis64;
   DevBuf<double> A64s, ilu64s;  // row-scaled operator / factor in SELL-64 order (FP64 Krylov)
   DevBuf<float> A32, ilu32s, iluy32, vbasis32, rhs32, d32;
-  DevBuf<double> gmH, gmh1, gmh2, gmcs, gmsn, gmg, gmy, gmpart;
+  DevBuf<double> gmH, gmh1, gmh2, gmcs, gmsn, gmg, gmsum, gmpart, gmpart2;
   Work<float> w32;
   Work<double> w64;
   bool ilu_ready = false;

@@ -80,7 +80,7 @@ __device__ __forceinline__ void write_partials(const double (&v)[NR], double *pa
 __device__ __forceinline__ bool idle(const KState *st) { return st->done != 0; }
 
 // stages that only store a total
-enum { STAGE_RR = 100, STAGE_GMSTART = 101, STAGE_DOT0 = 102 };
+enum { STAGE_RR = 100 };
 
 template <int NR, int STAGE>
 __global__ void __launch_bounds__(VB) k_finalize(const double *__restrict__ partials, int nparts, KState *st,
@@ -98,12 +98,6 @@ __global__ void __launch_bounds__(VB) k_finalize(const double *__restrict__ part
   if (threadIdx.x != 0) return;
   if constexpr (STAGE == STAGE_RR) {
     st->rr = tot[0];
-  } else if constexpr (STAGE == STAGE_GMSTART) {
-    st->rr = tot[0];
-    st->gm_inv = tot[0] > 0 ? 1.0 / sqrt(tot[0]) : 0.0;
-    st->gm_beta = sqrt(tot[0]);
-  } else if constexpr (STAGE == STAGE_DOT0) {
-    st->dots[0] = tot[0];
   } else {
     run_stage<STAGE>(st, tot);
   }
@@ -190,22 +184,6 @@ __global__ void __launch_bounds__(VB) k_sell_spmv(int64_t nrows, const int32_t *
   } else if constexpr (NDOT == 3) {
     double v[3] = {d0, d1, d2};
     write_partials<3>(v, partials);
-  }
-}
-
-// r = b - Ahat x with the SELL-64 operator (GMRES restarts)
-template <class VA, class V, class VXo>
-__global__ void __launch_bounds__(VB) k_sell_residual(int64_t nrows, const int32_t *__restrict__ sptr,
-                                                      const int32_t *__restrict__ col, const VA *__restrict__ val,
-                                                      const VXo *__restrict__ x, const V *__restrict__ b,
-                                                      V *__restrict__ r) {
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < nrows; i += (int64_t)gridDim.x * VB) {
-    const int64_t sl = i >> 6;
-    const int32_t p1 = sptr[sl + 1];
-    double acc = 0.0;
-#pragma unroll 4
-    for (int32_t q = sptr[sl] + (int32_t)(i & 63); q < p1; q += 64) acc += (double)val[q] * (double)x[col[q]];
-    r[i] = (V)((double)b[i] - acc);
   }
 }
 
@@ -468,143 +446,11 @@ __global__ void __launch_bounds__(VB) k_ilu_upper_sell(int32_t r0, int32_t r1, c
   z[perm[i]] = xv;
 }
 
-// ---------------------------------------------------------- GMRES ----------
-// h_j = (V_j, w) for j < k+1 (classical Gram-Schmidt, one pass): partials per j
-template <class V>
-__global__ void __launch_bounds__(VB) k_multidot(int64_t n, int nv, const V *__restrict__ Vb, int64_t ldv,
-                                                 const V *__restrict__ w, double *__restrict__ out_partials,
-                                                 const KState *st) {
-  if (idle(st)) return;
-  __shared__ double sh[16];
-  for (int j = 0; j < nv; j++) {
-    double d = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
-      d += (double)Vb[(int64_t)j * ldv + i] * (double)w[i];
-    double s = block_sum(d, sh);
-    if (threadIdx.x == 0) out_partials[(size_t)j * gridDim.x + blockIdx.x] = s;
-  }
-}
-
-// sums the multidot partials, stores h[0..nv-1] of column k (one block)
-__global__ void k_multidot_finish(int nv, int nblocks, const double *__restrict__ partials, double *__restrict__ h,
-                                  const KState *st) {
-  if (idle(st)) return;
-  const int j = threadIdx.x;
-  if (j >= nv) return;
-  double acc = 0.0;
-  for (int b = 0; b < nblocks; b++) acc += partials[(size_t)j * nblocks + b];
-  h[j] = acc;
-}
-
-// w -= sum_j h_j V_j (h_j from device); ||w||^2 reduced
-template <class V>
-__global__ void __launch_bounds__(VB) k_multiaxpy(int64_t n, int nv, const V *__restrict__ Vb, int64_t ldv,
-                                                  const double *__restrict__ h, V *__restrict__ w, double *partials,
-                                                  KState *st, int final_pass) {
-  if (idle(st)) return;
-  double d = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
-    double acc = (double)w[i];
-    for (int j = 0; j < nv; j++) acc -= h[j] * (double)Vb[(int64_t)j * ldv + i];
-    const V wv = (V)acc;
-    w[i] = wv;
-    d += (double)wv * (double)wv;
-  }
-  double vv[1] = {d};
-  write_partials<1>(vv, partials);
-}
-
-// x_out = alpha x_in (normalise the new Krylov vector)
-template <class V>
-__global__ void __launch_bounds__(VB) k_gmres_normalize(int64_t n, const V *__restrict__ w, V *__restrict__ vnext,
-                                                        const KState *st) {
-  if (idle(st)) return;
-  const double inv = st->gm_inv;
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
-    vnext[i] = (V)((double)w[i] * inv);
-}
-
-// x += sum_j y_j Z_j where Z_j = M^-1 V_j is applied afterwards: here w = sum_j y_j V_j
-template <class V>
-__global__ void __launch_bounds__(VB) k_gmres_combine(int64_t n, int k, const V *__restrict__ Vb, int64_t ldv,
-                                                      const double *__restrict__ y, V *__restrict__ w) {
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
-    double acc = 0.0;
-    for (int j = 0; j < k; j++) acc += y[j] * (double)Vb[(int64_t)j * ldv + i];
-    w[i] = (V)acc;
-  }
-}
-
+// x += z
 template <class VXo, class V>
 __global__ void __launch_bounds__(VB) k_axpy_out(int64_t n, VXo *__restrict__ x, const V *__restrict__ z) {
   for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
     x[i] = (VXo)((double)x[i] + (double)z[i]);
-}
-
-// one thread: Givens update of Hessenberg column k (h has k+2 entries: h_0..h_k from the
-// two CGS passes, h_{k+1} = ||w||), residual estimate, convergence flag.
-__global__ void k_gmres_givens(int k, int m, double *__restrict__ H, const double *__restrict__ h1,
-                               const double *__restrict__ h2, double *__restrict__ cs, double *__restrict__ sn,
-                               double *__restrict__ g, KState *st) {
-  if (idle(st) || threadIdx.x != 0) return;
-  double col[65];
-  for (int j = 0; j <= k; j++) col[j] = h1[j] + h2[j];
-  const double hn = sqrt(st->dots[0]);
-  col[k + 1] = hn;
-  st->gm_inv = hn > 0 ? 1.0 / hn : 0.0;
-  for (int j = 0; j < k; j++) {
-    const double t0 = cs[j] * col[j] + sn[j] * col[j + 1];
-    col[j + 1] = -sn[j] * col[j] + cs[j] * col[j + 1];
-    col[j] = t0;
-  }
-  const double a = col[k], b = col[k + 1], den = sqrt(a * a + b * b);
-  cs[k] = den > 0 ? a / den : 1.0;
-  sn[k] = den > 0 ? b / den : 0.0;
-  col[k] = den;
-  g[k + 1] = -sn[k] * g[k];
-  g[k] = cs[k] * g[k];
-  for (int j = 0; j <= k; j++) H[j * m + k] = col[j];
-  st->iters += 1;
-  st->gm_k = k + 1;
-  const double res = fabs(g[k + 1]);
-  st->rr = res * res;
-  if (res * res <= st->tol2) st->gm_conv = 1;
-  if (st->iters >= st->maxit) st->gm_stop = 1;
-  if (hn == 0.0) st->gm_conv = 1;  // lucky breakdown: exact solution in the subspace
-  if (st->gm_conv || st->gm_stop) st->done = 1;  // later kernels of this cycle return at entry
-}
-
-// back substitution for y (one thread), k = st->gm_k
-__global__ void k_gmres_solve(int m, const double *__restrict__ H, const double *__restrict__ g, double *__restrict__ y,
-                              KState *st) {
-  if (threadIdx.x != 0) return;
-  const int k = st->gm_k;
-  for (int i = k - 1; i >= 0; i--) {
-    double acc = g[i];
-    for (int j = i + 1; j < k; j++) acc -= H[i * m + j] * y[j];
-    y[i] = acc / H[i * m + i];
-  }
-  for (int i = k; i < m; i++) y[i] = 0.0;
-}
-
-// restart: w = r (scaled residual) -> beta = ||r||; V_0 = r / beta; g = beta e_1
-template <class V>
-__global__ void __launch_bounds__(VB) k_gmres_start_norm(int64_t n, const V *__restrict__ r, double *partials, KState *st) {
-  double d = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB)
-    d += (double)r[i] * (double)r[i];
-  double vv[1] = {d};
-  write_partials<1>(vv, partials);
-}
-
-__global__ void k_gmres_reset(int m, double *g, KState *st) {
-  if (threadIdx.x != 0) return;
-  for (int j = 0; j <= m; j++) g[j] = 0.0;
-  g[0] = st->gm_beta;
-  st->gm_k = 0;
-  st->gm_conv = (st->rr <= st->tol2) ? 1 : 0;
-  st->gm_stop = 0;
-  st->done = 0;
 }
 
 // Newton update: U -= damp * dU ; ||dU||_inf, ||U||_1 (src/vfvm_solver.jl:116-135)
@@ -689,6 +535,7 @@ __global__ void __launch_bounds__(VB) k_maxdiff(int64_t n, const double *__restr
 }
 
 #include "vfvm_bicgstab.h"
+#include "vfvm_gmres.h"
 
 // CSC gather: out[k] = J[perm[k]]
 __global__ void __launch_bounds__(VB) k_gather(int64_t n, const int32_t *__restrict__ perm, const double *__restrict__ J,
@@ -714,6 +561,10 @@ static unsigned grid_for(int64_t n, int per_thread_rows = 1) {
 // 18.6.  The products keep one row per thread as far as it goes (13.4 us with 1024 blocks and
 // 18.1 with 512, against 11.5).
 constexpr unsigned FOLD_BLOCKS = 512;
+// Blocks up to which every block of GMRES sums the previous kernel's partial dot products itself
+// (up to 64 sums; beyond, a launch with one block per sum goes before).  A step took, folded and
+// summed, 24.4 and 27.6 us with 66 blocks, 25.8 and 27.6 with 128, 32.8 and 29.3 with 259.
+constexpr int GM_FOLD = 128;
 static unsigned fold_blocks(int64_t n) { return std::min(grid_for(n), FOLD_BLOCKS); }
 
 void LinearSolver::setup(const LinSetup &ls, hipStream_t s) {
@@ -780,8 +631,9 @@ void LinearSolver::ensure_work(int precision, int krylov, int m) {
     gmcs.alloc((size_t)m);
     gmsn.alloc((size_t)m);
     gmg.alloc((size_t)m + 2);
-    gmy.alloc((size_t)m + 1);
+    gmsum.alloc((size_t)m + 2);
     gmpart.alloc((size_t)(m + 2) * MAX_RED_BLOCKS);
+    gmpart2.alloc((size_t)(m + 2) * GM_FOLD);
   }
 }
 
@@ -1243,82 +1095,125 @@ int LinearSolver::gmres(const VBin *b, VXo *x, const double *J, const vfvm_contr
   h.rtol = rtol;
   h.atol = atol;
   VFVM_HIP_CHECK(hipMemcpyAsync(st.p, &h, sizeof(KState), hipMemcpyHostToDevice, stream));
-  unsigned g = grid_for(n);
-  hipLaunchKernelGGL((k_fill<VXo>), dim3(g), dim3(VB), 0, stream, n, x, (VXo)0);
-  hipLaunchKernelGGL((k_convert<V, VBin>), dim3(g), dim3(VB), 0, stream, n, b, bb);
-  // tolerance from ||b||
-  hipLaunchKernelGGL((k_gmres_start_norm<V>), dim3(g), dim3(VB), 0, stream, n, bb, partials.p, st.p);
-  hipLaunchKernelGGL((k_finalize<1, STAGE_GMSTART>), dim3(1), dim3(VB), 0, stream, (const double *)partials.p, (int)g,
-                     st.p, 0);
-  read_state(h);
-  const double tol = atol + rtol * std::sqrt(h.rr);
-  h.tol2 = tol * tol;
-  h.rr0 = h.rr;
-  VFVM_HIP_CHECK(hipMemcpyAsync(st.p, &h, sizeof(KState), hipMemcpyHostToDevice, stream));
-  int status = VFVM_ERR_LINEAR;
-  while (true) {
-    // r = bhat - Ahat x
-    if constexpr (sizeof(V) == 4)
-      hipLaunchKernelGGL((k_sell_residual<float, V, VXo>), dim3(grid_for(n)), dim3(VB), 0, stream, n, L.sell_ptr,
-                         L.sell_col, (const float *)A32.p, x, bb, r);
-    else
-      hipLaunchKernelGGL((k_sell_residual<double, V, VXo>), dim3(grid_for(n)), dim3(VB), 0, stream, n, L.sell_ptr,
-                         L.sell_col, (const double *)A64s.p, x, bb, r);
-    hipLaunchKernelGGL((k_gmres_start_norm<V>), dim3(g), dim3(VB), 0, stream, n, r, partials.p, st.p);
-    hipLaunchKernelGGL((k_finalize<1, STAGE_GMSTART>), dim3(1), dim3(VB), 0, stream, (const double *)partials.p,
-                       (int)g, st.p, 0);
-    hipLaunchKernelGGL(k_gmres_reset, dim3(1), dim3(1), 0, stream, m, gmg.p, st.p);
-    hipLaunchKernelGGL((k_gmres_normalize<V>), dim3(g), dim3(VB), 0, stream, n, r, Vb, st.p);
-    read_state(h);
-    if (h.gm_conv) {
-      status = 0;
-      break;
+  const bool blk = c.precon == VFVM_PRECON_BLOCKJACOBI && L.nspec > 1;
+  const bool plain = c.precon == VFVM_PRECON_JACOBI || (c.precon == VFVM_PRECON_BLOCKJACOBI && L.nspec == 1);
+  const unsigned g = grid_for(n), gv = fold_blocks(n), gn = fold_blocks(L.nnodes);
+  const int kid = sizeof(V) == 4 ? VFVM_KERNEL_SPMV32 : VFVM_KERNEL_SPMV64;
+  const bool nt = sell_nt[sizeof(V) == 4 ? 0 : 1];
+  const V *val;
+  if constexpr (sizeof(V) == 4) val = A32.p;
+  else val = A64s.p;
+  GmArrays G{gmH.p, gmh1.p, gmh2.p, gmcs.p, gmsn.p, gmg.p, m};
+  int cur = 0, col = 0;  // slot of the current state; columns of the cycle
+  // v_k and z = M^-1 v_k from w after the norm partials in part_rho
+  auto next = [&](int k, bool first, int np, const V *from, KState *pinned) {
+    V *vk = Vb + (int64_t)(k + 1) * n;
+    auto go = [&](auto nsc) {
+      constexpr int NS = decltype(nsc)::value;
+      hipLaunchKernelGGL((k_gm_next<V, NS>), dim3(NS ? gn : gv), dim3(VB), 0, stream, NS ? L.nnodes : n, from, vk,
+                         (const double *)binv.p, z, G, k, first ? 1 : 0, (const double *)part_rho.p, np, st.p + cur,
+                         st.p + 1 - cur, pinned);
+    };
+    if (!blk) go(std::integral_constant<int, 0>());
+    else if (L.nspec == 2) go(std::integral_constant<int, 2>());
+    else go(std::integral_constant<int, 3>());
+    cur = 1 - cur;
+  };
+  // x += M^-1 (V y) and the state with no columns left
+  auto combine = [&]() {
+    auto go = [&](auto nsc, auto addc) {
+      constexpr int NS = decltype(nsc)::value;
+      hipLaunchKernelGGL((k_gm_combine<V, VXo, NS, decltype(addc)::value>), dim3(NS ? gn : gv), dim3(VB), 0, stream,
+                         NS ? L.nnodes : n, n, (const V *)Vb, (const double *)binv.p, w, x, G, st.p + cur,
+                         st.p + 1 - cur);
+    };
+    if (plain) {
+      go(std::integral_constant<int, 0>(), std::true_type());
+    } else if (blk) {
+      if (L.nspec == 2) go(std::integral_constant<int, 2>(), std::true_type());
+      else go(std::integral_constant<int, 3>(), std::true_type());
+    } else {
+      go(std::integral_constant<int, 0>(), std::false_type());
+      const V *zp = precond<V>(w, z, nullptr, 0, c);
+      hipLaunchKernelGGL((k_axpy_out<VXo, V>), dim3(g), dim3(VB), 0, stream, n, x, zp);
     }
-    if (h.iters >= maxit) break;
-    int k = 0;
-    for (; k < m; k++) {
-      V *vk = Vb + (int64_t)k * n, *vk1 = Vb + (int64_t)(k + 1) * n;
-      const V *zp = precond<V>(vk, z, nullptr, 0, c);
-      apply_op<V, 0, STAGE_NONE>(zp, w, (const V *)nullptr, nullptr, nullptr);
-      // CGS2: two passes of (h = V^T w ; w -= V h)
-      for (int pass = 0; pass < 2; pass++) {
-        double *hh = pass == 0 ? gmh1.p : gmh2.p;
-        hipLaunchKernelGGL((k_multidot<V>), dim3(g), dim3(VB), 0, stream, n, k + 1, Vb, n, w, gmpart.p, st.p);
-        hipLaunchKernelGGL(k_multidot_finish, dim3(1), dim3(64), 0, stream, k + 1, (int)g, gmpart.p, hh, st.p);
-        hipLaunchKernelGGL((k_multiaxpy<V>), dim3(g), dim3(VB), 0, stream, n, k + 1, Vb, n, hh, w, partials.p, st.p,
-                           pass);
-        if (pass == 1)
-          hipLaunchKernelGGL((k_finalize<1, STAGE_DOT0>), dim3(1), dim3(VB), 0, stream, (const double *)partials.p,
-                             (int)g, st.p, 1);
-      }
-      hipLaunchKernelGGL(k_gmres_givens, dim3(1), dim3(1), 0, stream, k, m, gmH.p, gmh1.p, gmh2.p, gmcs.p, gmsn.p,
-                         gmg.p, st.p);
-      hipLaunchKernelGGL((k_gmres_normalize<V>), dim3(g), dim3(VB), 0, stream, n, w, vk1, st.p);
-      if ((k + 1) % std::max(1, c.check_every) == 0 || k + 1 == m) {
-        read_state(h);
-        if (h.gm_conv || h.gm_stop) {
-          k++;
-          break;
-        }
-      }
+    cur = 1 - cur;
+  };
+  auto with_columns = [&](auto &&f) {
+    if (L.sell_off16 && sell16) f(L.sell_off16);
+    else f(L.sell_col);
+  };
+  auto step = [&](KState *pinned) {
+    if (col == m) {
+      combine();
+      with_columns([&](const auto *ci) {
+        using CI = std::remove_const_t<std::remove_pointer_t<decltype(ci)>>;
+        hipLaunchKernelGGL((k_gm_residual<V, VXo, CI>), dim3(g), dim3(VB), 0, stream, n, L.sell_ptr, ci, val,
+                           (const VXo *)x, (const V *)bb, r, (const KState *)(st.p + cur), part_rho.p);
+      });
+      next(-1, false, (int)g, r, nullptr);
+      col = 0;
     }
-    // x += M^-1 (V y)
-    hipLaunchKernelGGL(k_gmres_solve, dim3(1), dim3(1), 0, stream, m, gmH.p, gmg.p, gmy.p, st.p);
-    read_state(h);
-    hipLaunchKernelGGL((k_gmres_combine<V>), dim3(g), dim3(VB), 0, stream, n, h.gm_k, Vb, n, gmy.p, w);
-    const V *zp = precond<V>(w, z, nullptr, 0, c);
-    hipLaunchKernelGGL((k_axpy_out<VXo, V>), dim3(g), dim3(VB), 0, stream, n, x, zp);
+    const int k = col++, nv = k + 1;
+    KState *sk = st.p + cur;
+    const V *vk = Vb + (int64_t)k * n;
+    const V *zp = plain ? vk : blk ? (const V *)z : precond<V>(vk, z, sk, 0, c);
+    if (L.probe) L.probe->before(kid, stream);
+    with_columns([&](const auto *ci) {
+      using CI = std::remove_const_t<std::remove_pointer_t<decltype(ci)>>;
+      if (nt)
+        VFVM_LAUNCH((k_gm_av<V, true, CI>), dim3(g), dim3(VB), 0, stream, n, L.sell_ptr, ci, val, zp, w, nv,
+                    (const V *)Vb, gmpart.p, (const KState *)sk);
+      else
+        VFVM_LAUNCH((k_gm_av<V, false, CI>), dim3(g), dim3(VB), 0, stream, n, L.sell_ptr, ci, val, zp, w, nv,
+                    (const V *)Vb, gmpart.p, (const KState *)sk);
+    });
+    if (L.probe) L.probe->after(kid, stream, L.ndof, L.nnz);
+    const bool fold = (int)g <= GM_FOLD;
+    auto ortho = [&](auto lastc, const double *part, double *hout, double *pout) {
+      if (!fold)
+        hipLaunchKernelGGL(k_gm_sum, dim3(nv), dim3(VB), 0, stream, (int)g, part, gmsum.p, (const KState *)sk);
+      hipLaunchKernelGGL((k_gm_ortho<V, decltype(lastc)::value>), dim3(g), dim3(VB), 0, stream, n, nv, (const V *)Vb, w,
+                         fold ? part : (const double *)gmsum.p, fold ? (int)g : 1, hout, pout, (const KState *)sk);
+    };
+    double *second = fold ? gmpart2.p : gmpart.p;
+    ortho(std::false_type(), gmpart.p, gmh1.p, second);
+    ortho(std::true_type(), second, gmh2.p, part_rho.p);
+    next(k, false, (int)g, w, pinned);
+  };
+  hipLaunchKernelGGL((k_gm_init<V, VBin, VXo>), dim3(gv), dim3(VB), 0, stream, n, b, bb, x, part_rho.p);
+  next(-1, true, (int)gv, bb, nullptr);
+  // queued and polled as in bicgstab
+  const int every = std::max(1, c.check_every);
+  int launched = 0;
+  auto enqueue = [&](int nit, int slot) {
+    for (int q = 0; q < nit; q++) step(q == nit - 1 ? hst[slot] : nullptr);
     VFVM_HIP_CHECK(hipGetLastError());
-    if (h.gm_conv) {
-      status = 0;
-      break;
+    launched += nit;
+    VFVM_HIP_CHECK(hipEventRecord(sev[slot], stream));
+  };
+  int slot = 0, last = 0;
+  enqueue(std::max(every, std::min(maxit, last_iters - 1)), 0);
+  while (true) {
+    const bool more = launched < maxit + every;
+    if (more) {
+      enqueue(every, 1 - slot);
+      last = 1 - slot;
     }
-    if (h.iters >= maxit) break;
+    VFVM_HIP_CHECK(hipEventSynchronize(sev[slot]));
+    h = *hst[slot];
+    if (h.done || !more) break;
+    slot = 1 - slot;
   }
+  combine();  // of the cycle that the solve ended in, unless the queue has done it
+  VFVM_HIP_CHECK(hipGetLastError());
+  VFVM_HIP_CHECK(hipEventSynchronize(sev[last]));
+  h = *hst[last];
   iters = h.iters;
+  last_iters = h.iters;
   last_rr = h.rr;
   last_rr0 = h.rr0;
-  return status;
+  return h.gm_conv ? 0 : VFVM_ERR_LINEAR;
 }
 
 // Solve A x = b (b, x FP64 device vectors) with the prepared operator.
