@@ -91,6 +91,23 @@ def test_gradient_matches_oracle():
         assert np.linalg.norm(a - b) <= 3e-2 * max(np.linalg.norm(a), 1e-12)
 
 
+@pytest.mark.parametrize("n,nsamples", [(3, 1), (8, 1), (16, 1), (17, 3), (65, 32)])
+def test_gradient_matches_oracle_row_counts(n, nsamples):
+    """9, 64, 256, 867 and 135,200 rows: less than a tile, whole tiles and blocks, a partial last tile, more rows
+    than the blocks of the weight gradient take at least (the bounds are those of the test above: bfloat16
+    roundings of single activations)"""
+    print("case mpnn gradient", n, nsamples, flush=True)
+    net, graph, X, T = _setup(n=n, nsamples=nsamples, seed=4)
+    theta = net.params().astype(np.float64)
+    loss_g, grad_g = net.loss_grad(X, T)
+    loss_c, grad_c = M.loss_and_grad(theta, X.astype(np.float64), T.astype(np.float64), graph, nlayers=4,
+                                     emulate_bf16=True)
+    rel = np.linalg.norm(grad_g - grad_c) / np.linalg.norm(grad_c)
+    print("loss", loss_g, loss_c, "grad rel err", rel, flush=True)
+    assert abs(loss_g - loss_c) <= 1e-3 * abs(loss_c)
+    assert rel <= 2e-2
+
+
 def test_training_reduces_loss():
     print("case mpnn training", flush=True)
     net, graph, X, T = _setup(n=17, nsamples=8, seed=2)

@@ -70,7 +70,7 @@ enum { EPI_ENC = 0, EPI_RES = 1, EPI_DCAT = 2 };
 struct GemmEpi {
   const float *bias;  // ND (ENC, RES)
   float *hf;          // rows x 64 hidden state (ENC: written, RES: updated in place)
-  float *rbuf;        // rows x 64 relu(z) kept for the backward pass (RES)
+  uint8_t *gate;      // rows x 64: relu(z) > 0, kept for the backward pass (RES)
   bf16_t *cat;        // rows x 128: ENC/RES write bf(h) into cols 0..63 of the next layer input
   float *dh;          // DCAT: dh += dC[:, 0:64]
   float *da;          // DCAT: da  = dC[:, 64:128]
@@ -80,13 +80,25 @@ template <int KD, int ND, int EPI>
 __global__ void __launch_bounds__(TB) k_gemm(int64_t M, const bf16_t *__restrict__ A, const bf16_t *__restrict__ B,
                                              GemmEpi e) {
   constexpr int ASTR = KD + 8;
-  __shared__ bf16_t As[64 * ASTR];
-  __shared__ bf16_t Bs[KD * ND];
+  __shared__ alignas(16) bf16_t As[64 * ASTR];
+  __shared__ alignas(16) bf16_t Bs[KD * ND];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, c = l & 15;
   const int64_t row0 = (int64_t)blockIdx.x * 64;
-  for (int q = tid; q < KD * ND / 4; q += TB) {  // B: 4 bf16 per load
-    const uint64_t v = reinterpret_cast<const uint64_t *>(B)[q];
-    reinterpret_cast<uint64_t *>(Bs)[q] = v;
+  // B in operand order, one 8-byte fragment per k-step, column tile and lane: a thread transposes
+  // a 4 x 4 patch
+  for (int q = tid; q < KD * ND / 16; q += TB) {
+    const int kq = q / (ND / 4), cq = q % (ND / 4);
+    uint64_t v[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = reinterpret_cast<const uint64_t *>(B + (4 * kq + i) * ND)[cq];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      uint64_t o = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) o |= ((v[i] >> (16 * j)) & 0xffffull) << (16 * i);
+      const int col = 4 * cq + j;
+      reinterpret_cast<uint64_t *>(Bs)[((kq >> 2) * (ND / 16) + (col >> 4)) * 64 + (kq & 3) * 16 + (col & 15)] = o;
+    }
   }
   for (int q = tid; q < 64 * KD / 4; q += TB) {  // A tile rows, zero beyond M
     const int r = q / (KD / 4), kq = q % (KD / 4);
@@ -100,15 +112,10 @@ __global__ void __launch_bounds__(TB) k_gemm(int64_t M, const bf16_t *__restrict
   for (int t = 0; t < ND / 16; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int k0 = 0; k0 < KD; k0 += 16) {
-    bf16x4 a;
-    const bf16_t *ap = &As[(w * 16 + c) * ASTR + k0 + 4 * g];
-#pragma unroll
-    for (int j = 0; j < 4; j++) a[j] = (short)ap[j];
+    const bf16x4 a = *reinterpret_cast<const bf16x4 *>(&As[(w * 16 + c) * ASTR + k0 + 4 * g]);
 #pragma unroll
     for (int t = 0; t < ND / 16; t++) {
-      bf16x4 b;
-#pragma unroll
-      for (int j = 0; j < 4; j++) b[j] = (short)Bs[(k0 + 4 * g + j) * ND + t * 16 + c];
+      const bf16x4 b = reinterpret_cast<const bf16x4 *>(Bs)[((k0 >> 4) * (ND / 16) + t) * 64 + l];
       acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
     }
   }
@@ -126,7 +133,7 @@ __global__ void __launch_bounds__(TB) k_gemm(int64_t M, const bf16_t *__restrict
         if (e.cat) e.cat[row * CW + col] = f2bf(h);
       } else if constexpr (EPI == EPI_RES) {
         const float r = fmaxf(v + e.bias[col], 0.f);
-        e.rbuf[row * WID + col] = r;
+        e.gate[row * WID + col] = r > 0.f;
         const float hn = e.hf[row * WID + col] + r;
         e.hf[row * WID + col] = hn;
         if (e.cat) e.cat[row * CW + col] = f2bf(hn);
@@ -143,15 +150,39 @@ __global__ void __launch_bounds__(TB) k_gemm(int64_t M, const bf16_t *__restrict
 // Weight gradient: P_b[KD x 64] = sum over the block's rows of A[rows x KD]^T Z[rows x 64],
 // A and Z bfloat16.  Reduction over rows on the matrix cores (16 rows per step):
 // A-operand A'[k][m] = A[m][k] (m = row), B-operand Z[m][n].  Output tiles
-// (KD/16) x 4 are split over the 4 waves.
+// (KD/16) x 4 are split over the 4 waves.  Both operands want four consecutive rows of one
+// column per lane, so tiles are staged transposed: a thread loads a 4 x 4 patch (8 bytes of each
+// of 4 rows) and stores its columns, and an operand is one 8-byte LDS read (as 4 separate
+// 2-byte reads of untransposed tiles the kernel was bound by LDS).
+template <int KD>
+__device__ __forceinline__ void stage_transposed(int64_t r0, int64_t r_end, const bf16_t *__restrict__ A,
+                                                 bf16_t *__restrict__ T, int tstr) {
+  for (int q = threadIdx.x; q < 16 * (KD / 4); q += TB) {
+    const int rq = q / (KD / 4), kq = q % (KD / 4);
+    uint64_t v[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int64_t row = r0 + 4 * rq + i;
+      v[i] = row < r_end ? reinterpret_cast<const uint64_t *>(A + row * KD)[kq] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      uint64_t o = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) o |= ((v[i] >> (16 * j)) & 0xffffull) << (16 * i);
+      *reinterpret_cast<uint64_t *>(&T[(4 * kq + j) * tstr + 4 * rq]) = o;
+    }
+  }
+}
+
 template <int KD>
 __global__ void __launch_bounds__(TB) k_wgrad(int64_t M, int64_t rows_per_block, const bf16_t *__restrict__ A,
                                               const bf16_t *__restrict__ Z, float *__restrict__ partials) {
   constexpr int NT = (KD / 16) * (WID / 16);
   constexpr int PER = (NT + 3) / 4;
-  constexpr int ASTR = KD + 8, ZSTR = WID + 8;
-  __shared__ bf16_t As[64 * ASTR];
-  __shared__ bf16_t Zs[64 * ZSTR];
+  constexpr int STR = 64 + 4;  // rows of a tile, padded to spread the banks
+  __shared__ alignas(16) bf16_t As[KD * STR];
+  __shared__ alignas(16) bf16_t Zs[WID * STR];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, c = l & 15;
   f32x4 acc[PER];
 #pragma unroll
@@ -160,18 +191,8 @@ __global__ void __launch_bounds__(TB) k_wgrad(int64_t M, int64_t rows_per_block,
   const int64_t r_end = std::min<int64_t>(M, r_begin + rows_per_block);
   for (int64_t r0 = r_begin; r0 < r_end; r0 += 64) {
     __syncthreads();
-    for (int q = tid; q < 64 * KD / 4; q += TB) {
-      const int r = q / (KD / 4), kq = q % (KD / 4);
-      uint64_t v = 0;
-      if (r0 + r < r_end) v = reinterpret_cast<const uint64_t *>(A + (r0 + r) * KD)[kq];
-      *reinterpret_cast<uint64_t *>(&As[r * ASTR + kq * 4]) = v;
-    }
-    for (int q = tid; q < 64 * WID / 4; q += TB) {
-      const int r = q / (WID / 4), kq = q % (WID / 4);
-      uint64_t v = 0;
-      if (r0 + r < r_end) v = reinterpret_cast<const uint64_t *>(Z + (r0 + r) * WID)[kq];
-      *reinterpret_cast<uint64_t *>(&Zs[r * ZSTR + kq * 4]) = v;
-    }
+    stage_transposed<KD>(r0, r_end, A, As, STR);
+    stage_transposed<WID>(r0, r_end, Z, Zs, STR);
     __syncthreads();
 #pragma unroll
     for (int m0 = 0; m0 < 64; m0 += 16) {
@@ -180,12 +201,8 @@ __global__ void __launch_bounds__(TB) k_wgrad(int64_t M, int64_t rows_per_block,
         const int tile = w * PER + p;
         if (tile >= NT) break;
         const int kt = tile / (WID / 16), nt = tile % (WID / 16);
-        bf16x4 a, b;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          a[j] = (short)As[(m0 + 4 * g + j) * ASTR + kt * 16 + c];
-          b[j] = (short)Zs[(m0 + 4 * g + j) * ZSTR + nt * 16 + c];
-        }
+        const bf16x4 a = *reinterpret_cast<const bf16x4 *>(&As[(kt * 16 + c) * STR + m0 + 4 * g]);
+        const bf16x4 b = *reinterpret_cast<const bf16x4 *>(&Zs[(nt * 16 + c) * STR + m0 + 4 * g]);
         acc[p] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[p], 0, 0, 0);
       }
     }
@@ -201,41 +218,83 @@ __global__ void __launch_bounds__(TB) k_wgrad(int64_t M, int64_t rows_per_block,
   }
 }
 
-// grad[k] = sum over blocks of partials[b][k]
-__global__ void k_sum_partials(int nblocks, int len, const float *__restrict__ partials, float *__restrict__ grad) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= len) return;
+// grad[k] = sum over blocks of partials[b][k]; 64 columns per block, 16 threads each (one thread
+// per column waited for one load after the other: 130 us for 65 partials)
+constexpr int SP_LANES = 16;
+__global__ void __launch_bounds__(64 * SP_LANES) k_sum_partials(int nblocks, int len,
+                                                                const float *__restrict__ partials,
+                                                                float *__restrict__ grad) {
+  __shared__ float sh[SP_LANES][64];
+  const int c = threadIdx.x & 63, r = threadIdx.x >> 6, k = blockIdx.x * 64 + c;
   float acc = 0.f;
-  for (int b = 0; b < nblocks; b++) acc += partials[(size_t)b * len + k];
-  grad[k] = acc;
+  if (k < len)
+#pragma unroll 8
+    for (int b = r; b < nblocks; b += SP_LANES) acc += partials[(size_t)b * len + k];
+  sh[r][c] = acc;
+  __syncthreads();
+  if (r != 0 || k >= len) return;
+  float t = 0.f;
+#pragma unroll
+  for (int q = 0; q < SP_LANES; q++) t += sh[q][c];
+  grad[k] = t;
 }
 
 // ------------------------------------------------------------ graph ops ----
-// a_i = sum_j w_ij h_j - h_i for row r = s*n + i; one wave (64 features) per row
-__global__ void __launch_bounds__(TB) k_aggregate(int64_t rows, int64_t n, const int32_t *__restrict__ gptr,
+// Neighbour sums of a row's 4 features per lane (16 lanes and float4 a row, 4 rows a wave): the
+// sums are in the order of the row's entries, with the loads of 4 entries issued together.  `at`
+// is the sample's first row.
+__device__ __forceinline__ f32x4 neighbour_sum(int32_t k0, int32_t k1, const int32_t *__restrict__ gcol,
+                                               const float *__restrict__ gw, const float *__restrict__ h, uint32_t at,
+                                               int f) {
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int32_t k = k0; k < k1; k += 4) {
+    float w[4];
+    f32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {  // past the row's end: its last entry, not added
+      const int32_t q = std::min(k + j, k1 - 1);
+      w[j] = gw[q];
+      v[j] = *reinterpret_cast<const f32x4 *>(h + (size_t)(at + (uint32_t)gcol[q]) * WID + f);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (k + j < k1)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] += w[j] * v[j][e];
+  }
+  return acc;
+}
+
+// a_i = sum_j w_ij h_j - h_i for row r = s*n + i (rows < 2^32: the hidden state alone has 64
+// floats a row).  The wave-per-row form with its 64-bit division took 97 us for 266,256 rows of
+// a 2D grid, this one 25 us (with 68 MB read and 34 MB written: 20 us).
+__global__ void __launch_bounds__(TB) k_aggregate(uint32_t rows, uint32_t n, const int32_t *__restrict__ gptr,
                                                   const int32_t *__restrict__ gcol, const float *__restrict__ gw,
                                                   const float *__restrict__ hf, bf16_t *__restrict__ cat) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int f = threadIdx.x & 63;
+  const uint32_t row = blockIdx.x * (TB / 16) + (threadIdx.x >> 4);
+  const int f = 4 * (threadIdx.x & 15);
   if (row >= rows) return;
-  const int64_t s = row / n, i = row % n;
-  float acc = 0.f;
-  for (int32_t k = gptr[i]; k < gptr[i + 1]; k++) acc += gw[k] * hf[(s * n + gcol[k]) * WID + f];
-  acc -= hf[row * WID + f];
-  cat[row * CW + WID + f] = f2bf(acc);
+  const uint32_t i = row % n;
+  const f32x4 self = *reinterpret_cast<const f32x4 *>(hf + (size_t)row * WID + f);
+  const f32x4 acc = neighbour_sum(gptr[i], gptr[i + 1], gcol, gw, hf, row - i, f) - self;
+  bf16x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; e++) o[e] = (short)f2bf(acc[e]);
+  *reinterpret_cast<bf16x4 *>(cat + (size_t)row * CW + WID + f) = o;
 }
 
 // dh_k += sum_{i in N(k)} w_ik da_i - da_k  (transpose weights gwt on k's entries)
-__global__ void __launch_bounds__(TB) k_aggregate_t(int64_t rows, int64_t n, const int32_t *__restrict__ gptr,
+__global__ void __launch_bounds__(TB) k_aggregate_t(uint32_t rows, uint32_t n, const int32_t *__restrict__ gptr,
                                                     const int32_t *__restrict__ gcol, const float *__restrict__ gwt,
                                                     const float *__restrict__ da, float *__restrict__ dh) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int f = threadIdx.x & 63;
+  const uint32_t row = blockIdx.x * (TB / 16) + (threadIdx.x >> 4);
+  const int f = 4 * (threadIdx.x & 15);
   if (row >= rows) return;
-  const int64_t s = row / n, k = row % n;
-  float acc = 0.f;
-  for (int32_t q = gptr[k]; q < gptr[k + 1]; q++) acc += gwt[q] * da[(s * n + gcol[q]) * WID + f];
-  dh[row * WID + f] += acc - da[row * WID + f];
+  const uint32_t k = row % n;
+  const f32x4 self = *reinterpret_cast<const f32x4 *>(da + (size_t)row * WID + f);
+  f32x4 *d = reinterpret_cast<f32x4 *>(dh + (size_t)row * WID + f);
+  const f32x4 old = *d;
+  *d = old + (neighbour_sum(gptr[k], gptr[k + 1], gcol, gwt, da, row - k, f) - self);
 }
 
 // One hidden layer for inference, aggregation fused into the GEMM: for a tile of 64
@@ -256,7 +315,7 @@ __global__ void __launch_bounds__(TB, 4) k_layer_infer(int64_t rows, int64_t n, 
                                                     float *__restrict__ u) {
   constexpr int ASTR = CW + 8;  // bf16 per LDS row of the layer input
   constexpr int KS = CW / 16, NTL = WID / 16;
-  __shared__ bf16_t As[64 * ASTR];
+  __shared__ alignas(16) bf16_t As[64 * ASTR];
   __shared__ uint64_t Bf[KS * NTL * 64];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, c = l & 15;
   for (int q = tid; q < KS * NTL * 64; q += TB) {
@@ -669,69 +728,103 @@ __global__ void k_pack16(int64_t rows, const float *__restrict__ x, const float 
   x16[q] = k < NFEAT ? x[r * NFEAT + k] : P[(int64_t)(k - NFEAT) * rows + r];
 }
 
-// u_r = h_L[r] . wd + bd (one wave per row); optional loss: du = 2 (u - t) / count,
-// dh = du wd, per-block partials of sum (u-t)^2, sum du h (64) and sum du
+// u_r = h_L[r] . wd + bd (one wave per row), du = 2 (u - t) / count, dh = du wd; per-block
+// partials (float64) of sum du h (64), sum (u-t)^2 and sum du over DEC_ROWS rows
+constexpr int DEC_ROWS = 256;
 __global__ void __launch_bounds__(TB) k_decode(int64_t rows, const float *__restrict__ hf, const float *__restrict__ wd,
                                                const float *__restrict__ bd, float *__restrict__ u,
                                                const float *__restrict__ target, float inv_count,
-                                               float *__restrict__ dh, float *__restrict__ part) {
-  __shared__ float sh_loss[4], sh_du[4];
-  __shared__ float sh_g[4][WID];
+                                               float *__restrict__ dh, double *__restrict__ part) {
+  __shared__ double sh_s[4][2];
+  __shared__ double sh_g[4][WID];
   const int w = threadIdx.x >> 6, f = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + w;
-  float hv = 0.f, du = 0.f, lo = 0.f;
-  if (row < rows) {
-    hv = hf[row * WID + f];
-    float v = hv * wd[f];
+  const int64_t r0 = (int64_t)blockIdx.x * DEC_ROWS;
+  const int64_t r1 = std::min<int64_t>(rows, r0 + DEC_ROWS);
+  const float wf = wd[f], b0 = bd[0];
+  double g = 0.0, sd = 0.0, lo = 0.0;
+#pragma unroll 4
+  for (int64_t row = r0 + w; row < r1; row += 4) {
+    const float hv = hf[row * WID + f], t = target[row];
+    float v = hv * wf;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    const float uu = v + bd[0];
+    const float uu = v + b0;
     if (f == 0) u[row] = uu;
-    if (target) {
-      const float d = uu - target[row];
-      du = 2.f * d * inv_count;
-      lo = d * d;
-      dh[row * WID + f] = du * wd[f];
-    }
+    const float d = uu - t, du = 2.f * d * inv_count;
+    dh[row * WID + f] = du * wf;
+    g += (double)(du * hv);
+    lo += (double)(d * d);
+    sd += (double)du;
   }
-  if (!target) return;
-  sh_g[w][f] = du * hv;
+  sh_g[w][f] = g;
   if (f == 0) {
-    sh_loss[w] = lo;
-    sh_du[w] = du;
+    sh_s[w][0] = lo;
+    sh_s[w][1] = sd;
   }
   __syncthreads();
-  if (w == 0) {
-    float gsum = sh_g[0][f] + sh_g[1][f] + sh_g[2][f] + sh_g[3][f];
-    float *pb = part + (size_t)blockIdx.x * (WID + 2);
-    pb[f] = gsum;
-    if (f == 0) {
-      pb[WID] = sh_loss[0] + sh_loss[1] + sh_loss[2] + sh_loss[3];
-      pb[WID + 1] = sh_du[0] + sh_du[1] + sh_du[2] + sh_du[3];
-    }
-  }
+  double *pb = part + (size_t)blockIdx.x * (WID + 2);
+  if (w == 0) pb[f] = (sh_g[0][f] + sh_g[1][f]) + (sh_g[2][f] + sh_g[3][f]);
+  if (w == 1 && f < 2) pb[WID + f] = (sh_s[0][f] + sh_s[1][f]) + (sh_s[2][f] + sh_s[3][f]);
 }
 
-// dz = dh * (gate > 0) -> bfloat16; per-block column sums of dz (bias gradient)
-// gate is r_l (float) or, for the encoder, bf(h0) in the first half of cat_0
+// decoder gradient (wd, then bd) and the loss sum from the partials; one block per value
+__global__ void __launch_bounds__(TB) k_decode_sum(int nblocks, const double *__restrict__ part,
+                                                   float *__restrict__ grad, double *__restrict__ loss) {
+  __shared__ double sh[TB / 64];
+  double a = 0.0;
+#pragma unroll 4
+  for (int b = threadIdx.x; b < nblocks; b += TB) a += part[(size_t)b * (WID + 2) + blockIdx.x];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = a;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const double t = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  const int q = blockIdx.x;
+  if (q < WID) grad[q] = (float)t;
+  if (q == WID) loss[0] = t;
+  if (q == WID + 1) grad[WID] = (float)t;
+}
+
+// dz = dh where the gate is open -> bfloat16; per-block column sums of dz (bias gradient).  The
+// gate is the layer's byte per value or, for the encoder, bf(h0) > 0 in the first half of cat_0.
+// 16 lanes and 4 columns each per row.
 template <bool GATE_BF>
-__global__ void __launch_bounds__(TB) k_gate(int64_t rows, const float *__restrict__ dh, const float *__restrict__ gate,
-                                             const bf16_t *__restrict__ gate_bf, bf16_t *__restrict__ dzb,
-                                             float *__restrict__ part, int rows_per_block) {
-  __shared__ float sh[4][WID];
-  const int w = threadIdx.x >> 6, f = threadIdx.x & 63;
+__global__ void __launch_bounds__(TB) k_gate(int64_t rows, const float *__restrict__ dh,
+                                             const uint8_t *__restrict__ gate, const bf16_t *__restrict__ gate_bf,
+                                             bf16_t *__restrict__ dzb, float *__restrict__ part, int rows_per_block) {
+  constexpr int RL = TB / 16;
+  __shared__ f32x4 sh[RL][16];
+  const int w = threadIdx.x >> 4, q = threadIdx.x & 15, f = 4 * q;
   const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
   const int64_t r1 = std::min<int64_t>(rows, r0 + rows_per_block);
-  float acc = 0.f;
-  for (int64_t row = r0 + w; row < r1; row += 4) {
-    const bool on = GATE_BF ? (bf2f(gate_bf[row * CW + f]) > 0.f) : (gate[row * WID + f] > 0.f);
-    const float dz = on ? dh[row * WID + f] : 0.f;
-    dzb[row * WID + f] = f2bf(dz);
-    acc += dz;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int64_t row = r0 + w; row < r1; row += RL) {
+    const f32x4 d = *reinterpret_cast<const f32x4 *>(dh + row * WID + f);
+    bf16x4 o;
+    uint32_t gb = 0;
+    bf16x4 gh = {0, 0, 0, 0};
+    if constexpr (GATE_BF)
+      gh = *reinterpret_cast<const bf16x4 *>(gate_bf + row * CW + f);
+    else
+      gb = *reinterpret_cast<const uint32_t *>(gate + row * WID + f);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const bool on = GATE_BF ? bf2f((bf16_t)gh[e]) > 0.f : ((gb >> (8 * e)) & 0xffu) != 0;
+      const float dz = on ? d[e] : 0.f;
+      o[e] = (short)f2bf(dz);
+      acc[e] += dz;
+    }
+    *reinterpret_cast<bf16x4 *>(dzb + row * WID + f) = o;
   }
-  sh[w][f] = acc;
+  sh[w][q] = acc;
   __syncthreads();
-  if (w == 0) part[(size_t)blockIdx.x * WID + f] = sh[0][f] + sh[1][f] + sh[2][f] + sh[3][f];
+  if (w != 0) return;
+  f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < RL; k++) t += sh[k][q];
+  *reinterpret_cast<f32x4 *>(part + (size_t)blockIdx.x * WID + f) = t;
 }
 
 // Adam on the float32 parameters (t = step count, bias-corrected)
@@ -788,7 +881,9 @@ struct vfvm_mpnn {
   DevBuf<bf16_t> Web, Wb, WTb;  // encoder; layers (L x 128 x 64) and transposes (L x 64 x 128)
   // activations for a batch of `cap` rows
   int64_t cap = 0;
-  DevBuf<float> x, x16, hf, rbuf, dh, da, u, target, part, sm0, sm1;
+  DevBuf<float> x, x16, hf, dh, da, u, target, part, sm0, sm1;
+  DevBuf<uint8_t> gate;
+  DevBuf<double> dpart, dloss;
   DevBuf<bf16_t> xb, cat, dzb;
   // device features of the Dirichlet-sides family (2D): per node x, y and the distances
   // to the bounding-box sides (south, east, north, west); per-sample inputs
@@ -813,7 +908,7 @@ int mguard(vfvm_ctx *ctx, F &&f) {
   }
 }
 
-inline unsigned nb(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
+inline unsigned nb(int64_t n, int64_t t) { return (unsigned)((n + t - 1) / t); }
 
 void refresh_bf16(vfvm_mpnn &m) {
   hipStream_t st = m.ctx->stream;
@@ -836,7 +931,13 @@ inline int64_t sample_chunk(int64_t nsamples, int64_t n) {
   return std::max<int64_t>(1, (nsamples + nchunk - 1) / nchunk);
 }
 
-constexpr int64_t WG_ROWS = 4096;  // rows per block of the weight-gradient kernels
+// Blocks of the weight-gradient kernels: two per compute unit (with 4096 rows a block, 266,256 rows
+// gave 65 blocks and 418 us; now 37 us, of which 21 for 102 MB), but at least 256 rows, as each block writes a whole
+// gradient (32 KB) of partial sums.
+constexpr int64_t WG_BLOCKS = 512, WG_MIN_ROWS = 256;
+inline int64_t wgrad_rows(int64_t rows) {
+  return std::max<int64_t>(WG_MIN_ROWS, ((rows + WG_BLOCKS - 1) / WG_BLOCKS + 63) / 64 * 64);
+}
 constexpr int GATE_ROWS = 256;     // rows per block of the gate kernel
 
 void ensure_cap(vfvm_mpnn &m, int64_t rows) {
@@ -846,17 +947,18 @@ void ensure_cap(vfvm_mpnn &m, int64_t rows) {
   m.x16.alloc((size_t)rows * KPAD);
   m.xb.alloc((size_t)rows * KPAD);
   m.hf.alloc((size_t)rows * WID);
-  m.rbuf.alloc((size_t)rows * WID * L);
+  m.gate.alloc((size_t)rows * WID * L);
   m.dh.alloc((size_t)rows * WID);
   m.da.alloc((size_t)rows * WID);
   m.u.alloc((size_t)rows);
   m.target.alloc((size_t)rows);
   m.cat.alloc((size_t)rows * CW * (L + 1));
   m.dzb.alloc((size_t)rows * WID);
-  const int64_t p1 = nb(rows, 4) * (int64_t)(WID + 2);
-  const int64_t p2 = (int64_t)nb(rows, WG_ROWS) * CW * WID;
-  const int64_t p3 = (int64_t)nb(rows, GATE_ROWS) * WID;
-  m.part.alloc((size_t)std::max({p1, p2, p3}));
+  const int64_t p1 = std::min<int64_t>(WG_BLOCKS, nb(rows, WG_MIN_ROWS)) * CW * WID;
+  const int64_t p2 = (int64_t)nb(rows, GATE_ROWS) * WID;
+  m.part.alloc((size_t)std::max(p1, p2));
+  m.dpart.alloc((size_t)nb(rows, DEC_ROWS) * (WID + 2));
+  m.dloss.alloc(1);
   m.cap = rows;
 }
 
@@ -1024,12 +1126,12 @@ void forward(vfvm_mpnn &m, int64_t rows) {
                      (const bf16_t *)m.Web.p, e);
   for (int l = 0; l < L; l++) {
     bf16_t *cl = m.cat.p + (size_t)l * rows * CW;
-    hipLaunchKernelGGL(k_aggregate, dim3(nb(rows, 4)), dim3(TB), 0, st, rows, m.n, (const int32_t *)m.gptr.p,
+    hipLaunchKernelGGL(k_aggregate, dim3(nb(rows, TB / 16)), dim3(TB), 0, st, (uint32_t)rows, (uint32_t)m.n, (const int32_t *)m.gptr.p,
                        (const int32_t *)m.gcol.p, (const float *)m.gw.p, (const float *)m.hf.p, cl);
     GemmEpi r{};
     r.bias = m.theta.p + m.off_b[l];
     r.hf = m.hf.p;
-    r.rbuf = m.rbuf.p + (size_t)l * rows * WID;
+    r.gate = m.gate.p + (size_t)l * rows * WID;
     r.cat = m.cat.p + (size_t)(l + 1) * rows * CW;  // next layer's h half (cat_L unused by the decoder)
     hipLaunchKernelGGL((k_gemm<CW, WID, EPI_RES>), dim3(nb(rows, 64)), dim3(TB), 0, st, rows, (const bf16_t *)cl,
                        (const bf16_t *)(m.Wb.p + (size_t)l * CW * WID), r);
@@ -1066,57 +1168,47 @@ void forward_infer(vfvm_mpnn &m, int64_t rows) {
 float backward(vfvm_mpnn &m, int64_t rows) {
   hipStream_t st = m.ctx->stream;
   const int L = m.nlayers;
-  const unsigned dblk = nb(rows, 4);
+  const unsigned dblk = nb(rows, DEC_ROWS);
   hipLaunchKernelGGL(k_decode, dim3(dblk), dim3(TB), 0, st, rows, (const float *)m.hf.p,
                      (const float *)m.theta.p + m.off_wd, (const float *)m.theta.p + m.off_bd, m.u.p,
-                     (const float *)m.target.p, 1.0f / (float)rows, m.dh.p, m.part.p);
-  // decoder gradient and loss from the per-block partials (64 + 2 per block)
-  std::vector<float> hpart((size_t)dblk * (WID + 2));
-  VFVM_HIP_CHECK(hipMemcpyAsync(hpart.data(), m.part.p, hpart.size() * sizeof(float), hipMemcpyDeviceToHost, st));
-  VFVM_HIP_CHECK(hipStreamSynchronize(st));
-  std::vector<double> gwd(WID, 0.0);
-  double loss = 0.0, gbd = 0.0;
-  for (unsigned b = 0; b < dblk; b++) {
-    for (int f = 0; f < WID; f++) gwd[f] += hpart[(size_t)b * (WID + 2) + f];
-    loss += hpart[(size_t)b * (WID + 2) + WID];
-    gbd += hpart[(size_t)b * (WID + 2) + WID + 1];
-  }
-  std::vector<float> gdec(WID + 1);
-  for (int f = 0; f < WID; f++) gdec[f] = (float)gwd[f];
-  gdec[WID] = (float)gbd;
-  VFVM_HIP_CHECK(hipMemcpyAsync(m.grad.p + m.off_wd, gdec.data(), (WID + 1) * sizeof(float), hipMemcpyHostToDevice, st));
-  VFVM_HIP_CHECK(hipStreamSynchronize(st));  // gdec is a local
-  const unsigned wg_blocks = nb(rows, WG_ROWS);
+                     (const float *)m.target.p, 1.0f / (float)rows, m.dh.p, m.dpart.p);
+  hipLaunchKernelGGL(k_decode_sum, dim3(WID + 2), dim3(TB), 0, st, (int)dblk, (const double *)m.dpart.p,
+                     m.grad.p + m.off_wd, m.dloss.p);
+  const int64_t wg_rows = wgrad_rows(rows);
+  const unsigned wg_blocks = nb(rows, wg_rows);
   const unsigned gate_blocks = nb(rows, GATE_ROWS);
   for (int l = L - 1; l >= 0; l--) {
     const bf16_t *cl = m.cat.p + (size_t)l * rows * CW;
     hipLaunchKernelGGL((k_gate<false>), dim3(gate_blocks), dim3(TB), 0, st, rows, (const float *)m.dh.p,
-                       (const float *)m.rbuf.p + (size_t)l * rows * WID, (const bf16_t *)nullptr, m.dzb.p, m.part.p,
+                       (const uint8_t *)m.gate.p + (size_t)l * rows * WID, (const bf16_t *)nullptr, m.dzb.p, m.part.p,
                        GATE_ROWS);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(WID), 0, st, (int)gate_blocks, WID, (const float *)m.part.p,
+    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(64 * SP_LANES), 0, st, (int)gate_blocks, WID, (const float *)m.part.p,
                        m.grad.p + m.off_b[l]);
-    hipLaunchKernelGGL((k_wgrad<CW>), dim3(wg_blocks), dim3(TB), 0, st, rows, WG_ROWS, cl, (const bf16_t *)m.dzb.p,
+    hipLaunchKernelGGL((k_wgrad<CW>), dim3(wg_blocks), dim3(TB), 0, st, rows, wg_rows, cl, (const bf16_t *)m.dzb.p,
                        m.part.p);
-    hipLaunchKernelGGL(k_sum_partials, dim3(nb(CW * WID, 256)), dim3(256), 0, st, (int)wg_blocks, CW * WID,
+    hipLaunchKernelGGL(k_sum_partials, dim3(CW * WID / 64), dim3(64 * SP_LANES), 0, st, (int)wg_blocks, CW * WID,
                        (const float *)m.part.p, m.grad.p + m.off_W[l]);
     GemmEpi e{};
     e.dh = m.dh.p;
     e.da = m.da.p;
     hipLaunchKernelGGL((k_gemm<WID, CW, EPI_DCAT>), dim3(nb(rows, 64)), dim3(TB), 0, st, rows, (const bf16_t *)m.dzb.p,
                        (const bf16_t *)(m.WTb.p + (size_t)l * CW * WID), e);
-    hipLaunchKernelGGL(k_aggregate_t, dim3(nb(rows, 4)), dim3(TB), 0, st, rows, m.n, (const int32_t *)m.gptr.p,
+    hipLaunchKernelGGL(k_aggregate_t, dim3(nb(rows, TB / 16)), dim3(TB), 0, st, (uint32_t)rows, (uint32_t)m.n, (const int32_t *)m.gptr.p,
                        (const int32_t *)m.gcol.p, (const float *)m.gwt.p, (const float *)m.da.p, m.dh.p);
   }
   // encoder: gate from bf(h0) in cat_0
   hipLaunchKernelGGL((k_gate<true>), dim3(gate_blocks), dim3(TB), 0, st, rows, (const float *)m.dh.p,
-                     (const float *)nullptr, (const bf16_t *)m.cat.p, m.dzb.p, m.part.p, GATE_ROWS);
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(WID), 0, st, (int)gate_blocks, WID, (const float *)m.part.p,
+                     (const uint8_t *)nullptr, (const bf16_t *)m.cat.p, m.dzb.p, m.part.p, GATE_ROWS);
+  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(64 * SP_LANES), 0, st, (int)gate_blocks, WID, (const float *)m.part.p,
                      m.grad.p + m.off_be);
-  hipLaunchKernelGGL((k_wgrad<KPAD>), dim3(wg_blocks), dim3(TB), 0, st, rows, WG_ROWS, (const bf16_t *)m.xb.p,
+  hipLaunchKernelGGL((k_wgrad<KPAD>), dim3(wg_blocks), dim3(TB), 0, st, rows, wg_rows, (const bf16_t *)m.xb.p,
                      (const bf16_t *)m.dzb.p, m.part.p);
-  hipLaunchKernelGGL(k_sum_partials, dim3(nb(KPAD * WID, 256)), dim3(256), 0, st, (int)wg_blocks, KPAD * WID,
+  hipLaunchKernelGGL(k_sum_partials, dim3(KPAD * WID / 64), dim3(64 * SP_LANES), 0, st, (int)wg_blocks, KPAD * WID,
                      (const float *)m.part.p, m.grad.p + m.off_We);
   VFVM_HIP_CHECK(hipGetLastError());
+  double loss = 0.0;
+  VFVM_HIP_CHECK(hipMemcpyAsync(&loss, m.dloss.p, sizeof(double), hipMemcpyDeviceToHost, st));
+  VFVM_HIP_CHECK(hipStreamSynchronize(st));
   return (float)(loss / (double)rows);
 }
 
