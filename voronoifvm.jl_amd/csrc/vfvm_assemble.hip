@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_assemble(AsmArgs a) {
             const double dk = g[i].d[j], dl = g[i].d[NS + j];
             bad |= (dk != dk) | (dl != dl);
             Jd[i][j] += f * dk;
-            a.J[boff + rank_in<NS>(em, j)] = f * dl;
+            a.J[boff + rank_in<NS>(em, j)] = a.jsign * (f * dl);
           }
         }
       }
@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_assemble(AsmArgs a) {
     double Fn[NS], Jn[NS][NS], Fb[NS], Jb[NS];
     node_terms<NS, JAC>(a, P, p, K, uK, uo, srcv, vol, bb0, bb1, Fn, Jn, Fb, Jb, bad);
 #pragma unroll
-    for (int i = 0; i < NS; i++) a.F[K * NS + i] = (Fn[i] + Fe[i]) + Fb[i];
+    for (int i = 0; i < NS; i++) a.F[K * NS + i] = a.fsign * ((Fn[i] + Fe[i]) + Fb[i]);
     if constexpr (JAC) {
 #pragma unroll
       for (int i = 0; i < NS; i++) {
@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_assemble(AsmArgs a) {
           if (dm & (1u << j)) {
             double v = Jn[i][j] + Jd[i][j];
             if (i == j) v += Jb[i];
-            a.J[boff + rank_in<NS>(dm, j)] = v;
+            a.J[boff + rank_in<NS>(dm, j)] = a.jsign * v;
           }
         }
       }
@@ -346,9 +346,9 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_assemble_stream(AsmArgs a) {
       rowbase[i] = (int64_t)(a0 - K) * a.m.etot + K * a.m.dtot + (int64_t)(deg1 - 1) * a.m.eoff[i] + a.m.doff[i];
     auto put = [&](int64_t slot, double v) {
       if (sJ)
-        s_J[slot - j0] = v;
+        s_J[slot - j0] = a.jsign * v;
       else
-        a.J[slot] = v;
+        a.J[slot] = a.jsign * v;
     };
     double Fe[NS], Jd[NS][NS];
 #pragma unroll
@@ -426,7 +426,7 @@ __global__ void __launch_bounds__(ASM_BLOCK) k_assemble_stream(AsmArgs a) {
     double Fn[NS], Jn[NS][NS], Fb[NS], Jb[NS];
     node_terms<NS, JAC>(a, P, p, K, uK, uo, srcv, vol, bb0, bb1, Fn, Jn, Fb, Jb, bad);
 #pragma unroll
-    for (int i = 0; i < NS; i++) a.F[K * NS + i] = (Fn[i] + Fe[i]) + Fb[i];
+    for (int i = 0; i < NS; i++) a.F[K * NS + i] = a.fsign * ((Fn[i] + Fe[i]) + Fb[i]);
     if constexpr (JAC) {
 #pragma unroll
       for (int i = 0; i < NS; i++) {

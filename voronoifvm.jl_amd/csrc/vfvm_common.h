@@ -235,6 +235,7 @@ struct AsmArgs {
   int32_t *flags;                // [0] NaN seen
   Masks m;
   int nspec;
+  double fsign = 1.0, jsign = 1.0;  // F and J are written times these (+1 or -1)
 };
 void launch_assemble(const AsmArgs &a, int group, hipStream_t s);
 // Compact form of a node graph (adj_ptr rows, adj_col, adj_fac): off[q] = adj_col[q] - row
