@@ -1,5 +1,5 @@
-"""The forms of the single-system BiCGStab (fused point Jacobi, block Jacobi, two-colour and general ILU(0)) and GMRES, with the
-sizes at which each changes): the row-scaled residual of the returned solution against the Jacobian on the host."""
+"""The forms of the single-system BiCGStab (one block, fused point Jacobi, block Jacobi, two-colour and general
+ILU(0)) and of GMRES, at the sizes where each changes: the row-scaled residual of the returned solution against the Jacobian on the host."""
 import numpy as np
 import pytest
 
@@ -27,8 +27,9 @@ def _system(name):
     return cases.pair(g, ns, data, [vfvm.Dirichlet(1, 1, 0.3)], oracle=False)[0], 1.0
 
 
-@pytest.mark.parametrize("name", ["grid:2", "grid:3", "grid:65", "grid:129", "grid:16:17", "grid:9:9:9", "grid:65:65:65",
-                                  "grid:70001:3", "exchange:17:9", "dd2d:9"])
+@pytest.mark.parametrize("name", ["grid:2", "grid:3", "grid:65", "grid:32:32", "grid:1025", "grid:2049", "grid:45:45",
+                                  "grid:9:9:9", "grid:50:50", "grid:3072", "grid:3073", "grid:70:70", "grid:6144", "grid:6145",
+                                  "grid:129:129", "grid:65:65:65", "grid:70001:3", "exchange:17:9", "dd2d:9"])
 @pytest.mark.parametrize("precon", ["jacobi", "blockjacobi", "ilu0"])
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_solution_meets_the_tolerance(name, precon, precision):

@@ -27,8 +27,8 @@ struct KState {
 // solver that computes s inside the second operator application
 enum { STAGE_NONE = 0, STAGE_INIT, STAGE_ALPHA, STAGE_SNORM, STAGE_OMEGA, STAGE_XR, STAGE_SOMEGA };
 
-template <int STAGE>
-__device__ __forceinline__ void run_stage(KState *st, const double *tot) {
+template <int STAGE, class S>
+__device__ __forceinline__ void run_stage(S *st, const double *tot) {
   if constexpr (STAGE == STAGE_INIT) {
     st->rr = tot[0];
     st->rr0 = tot[0];

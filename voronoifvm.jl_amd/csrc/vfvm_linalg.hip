@@ -535,6 +535,7 @@ __global__ void __launch_bounds__(VB) k_maxdiff(int64_t n, const double *__restr
 }
 
 #include "vfvm_bicgstab.h"
+#include "vfvm_bicgone.h"
 #include "vfvm_gmres.h"
 
 // CSC gather: out[k] = J[perm[k]]
@@ -851,6 +852,13 @@ void LinearSolver::prepare_red_black(const double *J, bool fp32) {
 // the same from 363^2 on (23.9 and 24.2; 51^3: 29.1 and 29.6; 513^2: 31.9 and 31.8).
 constexpr int64_t FUSE_P_ROWS = 1 << 17;
 
+// Matrix entries (with two colours: of the black rows) up to which one block solves the whole
+// system.  An iteration takes, in one block and in launches: point Jacobi 4.6 and 12 us at 33^2 rows
+// (7,700 entries, copied to LDS), 7.6 and 12 at 45^2, 10.1 and 12 at 55^2 (21,500), 12.7 and 12 at
+// 64^2 (29,000), 23.6 and 15.9 at 16^3; two-colour ILU(0) 3.9 and 15 us at 33^2 rows, 6.1 and 20 at
+// 45^2, 14 and 24 at 55^2, 20.7 and 24 at 71^2 (10,200), 29 and 24 at 80^2 (13,000).
+constexpr int64_t ONE_ENTRIES = 22000, ONE_ENTRIES_RB = 11000;
+
 // The launches of BiCGStab in the form that fits the preconditioner.  init() sets the start
 // state (slot 0 and the partials of (r, r)), iterate(first) queues one iteration, report() the
 // host's copy of the state after it.
@@ -974,8 +982,8 @@ struct LinearSolver::Bicg {
     }
     nrho = (int)gv;
   }
-  template <int STAGE, class CI>
-  void iterate_rb(const CI *ec, const CI *fc) {
+  template <class CI>
+  RbMat<V, CI> rb_matrix(const CI *ec, const CI *fc) {
     const RedBlack &R = S.L.ilu->rb;
     RbMat<V, CI> A;
     A.nr = R.nr;
@@ -993,6 +1001,61 @@ struct LinearSolver::Bicg {
       A.fv = S.rb_f64.p;
       A.d = S.rb_d64.p;
     }
+    return A;
+  }
+  // whole solve in one block: point Jacobi, two-colour ILU(0)
+  bool one_block() const {
+    if (rb) {
+      const RedBlack &R = S.L.ilu->rb;
+      return std::max(R.nr, R.nb) <= 3 * ONE_T && R.f.nval <= ONE_ENTRIES_RB;
+    }
+    return plain && n <= 3 * ONE_T && S.L.sell_nnz <= ONE_ENTRIES;
+  }
+  template <class VBin>
+  void solve_one(const VBin *b, const KState &h, int every, int stag, KState *pinned) {
+    auto go = [&](auto rc, auto cc) {
+      constexpr int R = decltype(rc)::value;
+      constexpr bool COPY = decltype(cc)::value;
+      if (rb) {
+        const RedBlack &B = S.L.ilu->rb;
+        auto launch = [&](const auto *ec, const auto *fc) {
+          using CI = std::remove_const_t<std::remove_pointer_t<decltype(ec)>>;
+          hipLaunchKernelGGL((k_rb_one<V, VBin, VXo, CI, R, COPY>), dim3(1), dim3(ONE_T), 0, st, rb_matrix<CI>(ec, fc),
+                             B.e.row, B.f.row, b, x, xx, r0, h.rtol, h.atol, h.maxit, every, stag, pinned);
+        };
+        if (B.e.off && B.f.off) launch(B.e.off, B.f.off);
+        else launch(B.e.col, B.f.col);
+      } else {
+        with_operator([&](auto, const auto *col, const V *val) {
+          using CI = std::remove_const_t<std::remove_pointer_t<decltype(col)>>;
+          const OneMat<V, CI> A{S.L.sell_ptr, col, val};
+          hipLaunchKernelGGL((k_bicg_one<V, VBin, VXo, CI, R, COPY>), dim3(1), dim3(ONE_T), 0, st, (int)n, A, b, x, r0,
+                             h.rtol, h.atol, h.maxit, every, stag, pinned);
+        });
+      }
+    };
+    int64_t m = n, bytes;
+    const int vs = sizeof(V);
+    if (rb) {
+      const RedBlack &R = S.L.ilu->rb;
+      const int cs = R.e.off && R.f.off ? 2 : 4;
+      m = std::max(R.nr, R.nb);
+      bytes = one_bytes(R.nr, R.e.nval, vs, cs) + one_bytes(R.nb, R.f.nval, vs, cs);
+    } else {
+      bytes = one_bytes(n, S.L.sell_nnz, vs, S.L.sell_off16 && S.sell16 ? 2 : 4);
+    }
+    auto rows = [&](auto cc) {
+      if (m <= ONE_T) go(std::integral_constant<int, 1>(), cc);
+      else if (m <= 2 * ONE_T) go(std::integral_constant<int, 2>(), cc);
+      else go(std::integral_constant<int, 3>(), cc);
+    };
+    if (bytes <= ONE_LDS) rows(std::true_type());
+    else rows(std::false_type());
+  }
+  template <int STAGE, class CI>
+  void iterate_rb(const CI *ec, const CI *fc) {
+    const RedBlack &R = S.L.ilu->rb;
+    const RbMat<V, CI> A = rb_matrix<CI>(ec, fc);
     KState *k0 = k + SLOT_RHO, *k1 = k + SLOT_BETA, *k2 = k + SLOT_ALPHA;
     const unsigned gr = grid_for(R.nr), gb = grid_for(R.nb);
     const int np = (int)(gr + gb);
@@ -1028,8 +1091,20 @@ int LinearSolver::bicgstab(const VBin *b, VXo *x, const double *J, const vfvm_co
   h.maxit = maxit;
   h.rtol = rtol;
   h.atol = atol;
-  VFVM_HIP_CHECK(hipMemcpyAsync(st.p, &h, sizeof(KState), hipMemcpyHostToDevice, stream));
   Bicg<V, VXo> K(*this, c, x);
+  if (K.one_block()) {
+    K.solve_one(b, h, std::max(1, c.check_every), stag_window, hst[0]);
+    VFVM_HIP_CHECK(hipGetLastError());
+    VFVM_HIP_CHECK(hipEventRecord(sev[0], stream));
+    VFVM_HIP_CHECK(hipEventSynchronize(sev[0]));
+    h = *hst[0];
+    iters = h.iters;
+    last_iters = h.iters;
+    last_rr = h.rr;
+    last_rr0 = h.rr0;
+    return h.status == 1 ? 0 : VFVM_ERR_LINEAR;
+  }
+  VFVM_HIP_CHECK(hipMemcpyAsync(st.p, &h, sizeof(KState), hipMemcpyHostToDevice, stream));
   K.init(b);
   // first chunk: about as many iterations as the previous solve needed (Newton steps of one
   // solve need similar counts), then poll every check_every iterations
