@@ -105,3 +105,25 @@ def test_batch_sell_index_widths_agree(precision):
         assert it == out[0][1]
         for a, b in zip(U, out[0][0]):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("check_every", [1, 3, 8])
+@pytest.mark.parametrize("sizes", [(2, 511, 512, 513), (1025, 3, 33000)])
+def test_batch_members_at_chunk_edges(sizes, check_every):
+    """Members of one row to more than 64 chunks, whole and partial last chunks, odd and even polling blocks, as
+    graphs and as launches: the Newton solutions are the oracle's (its direct solves; both stop at 1e-10 of the
+    first update)."""
+    print("case batch chunks", sizes, check_every, flush=True)
+    pairs = []
+    for k, n in enumerate(sizes):
+        g = vfvm.simplexgrid(vfvm.linspace(0.0, 1.0, n))
+        h2 = 1.0 / (n - 1) ** 2  # diffusion as large as the reaction (whose slope is at least 1)
+        pairs.append(cases.pair(g, 1, dict(flux=vfvm.LinearFlux(h2), reaction=vfvm.SinhReaction()),
+                                [vfvm.Dirichlet(1, 1, 0.2 + 0.1 * k), vfvm.Dirichlet(1, 2, 0.5)]))
+    ctrl = vfvm.SolverControl(reltol_linear=1e-12, abstol_linear=0.0, maxiters_linear=4000, check_every=check_every)
+    batch = vfvm.Batch([p[0] for p in pairs])
+    for graphs in (False, True):
+        batch.set_graphs(graphs)
+        for (s, o), U in zip(pairs, batch.solve(0.5, ctrl)):
+            Uo, _ = o.solve_step(np.full(s.grid.num_nodes, 0.5))
+            assert np.abs(vfvm.dofs(U) - Uo).max() <= 1e-9

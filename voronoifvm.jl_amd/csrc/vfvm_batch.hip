@@ -7,9 +7,9 @@
 // node carries its member index (node_inst) and the assembly kernel reads the
 // member's parameters and boundary table from a per-member block.  The Krylov
 // kernels work on "chunks" of at most CHUNK rows that never straddle two
-// members; every reduction writes per-chunk partials and a finalize kernel with
-// one block per member sums them and updates that member's solver scalars.  Converged members drop
-// out: their kernels return at entry and their nodes are skipped by assembly.
+// members; every reduction writes per-chunk partials, which the next kernel (point Jacobi
+// BiCGStab) or a finalize kernel with one block per member sums to update that member's
+// solver scalars.  Converged members drop out: their kernels return at entry and their nodes are skipped by assembly.
 // One launch therefore advances every unfinished member, whatever its size.
 #include <hip/hip_runtime.h>
 
@@ -24,6 +24,7 @@
 
 #include "vfvm_amg_dev.h"
 #include "vfvm_sys.h"
+#include "vfvm_wave.h"
 
 using namespace vfvm;
 
@@ -42,8 +43,7 @@ struct Seg {
 };
 
 __device__ __forceinline__ double bsum(double v, double *sh) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -117,6 +117,7 @@ __global__ void __launch_bounds__(BB) k_bfinalize(Seg S, KState *st, const int32
     sti->rr = tot[0];
   } else if constexpr (MODE == BF_INIT) {
     run_stage<STAGE_INIT>(sti, tot);
+    sti->pad = 1;  // no iteration yet
     if (active && !active[m]) {
       sti->done = 1;
       sti->status = 1;
@@ -177,53 +178,228 @@ __global__ void __launch_bounds__(BB) k_bspmv(Seg S, const int32_t *__restrict__
   }
 }
 
-// The BiCGStab half step and the second operator application in one launch:
-// s = r - alpha v for the chunk's rows (written) and, for every column the SpMV
-// gathers, recomputed from r and v with the same fused multiply-add, t = Ahat s,
-// and the dots (s, t), (t, t), (s, s) for STAGE_SOMEGA.
+// ---- point Jacobi BiCGStab, one launch per Krylov step ----
+//
+// Three kernels an iteration.  The reductions have no launches: a kernel writes one partial per
+// chunk, and every chunk of the next kernel sums its member's partials (at most a few hundred) in
+// the same order and runs the stage on its copy of the member's state.  The state moves through
+// three arrays (st -> s1 -> s2 -> st), so no chunk reads what another one is writing; the member's
+// first chunk stores it.  p' = r + beta (p - omega v) and s = r - alpha v are formed again for
+// every gathered column, with the same rounding, instead of taking a pass of their own.
+// KState::pad marks a state before its first iteration.
+//
+// 64 uneven members of up to 257^2 rows: 52 us an iteration in seven launches (products 15 and 12,
+// update 8, direction 5, three sums of 4 and more), 33 in three.
+// Workgroups are dealt to the 8 XCDs in turn.  A chunk's rows gather from the chunks beside it, so
+// XCHUNK neighbouring chunks go to one XCD and its L2 (and the next ones to the next, which keeps
+// all of them busy when few members are left).  -1: past the last chunk.
+constexpr int XCHUNK = 8;
+__device__ __forceinline__ int chunk_of(const Seg &S) {
+  const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int64_t c = (int64_t)(j / XCHUNK) * (8 * XCHUNK) + x * XCHUNK + j % XCHUNK;
+  return c < S.nch ? (int)c : -1;
+}
+inline unsigned chunk_grid(int64_t nch) { return (unsigned)((nch + 8 * XCHUNK - 1) / (8 * XCHUNK) * (8 * XCHUNK)); }
+
+template <int STAGE, int NR>
+struct BFold {
+  double a[NR];
+  // `part`: NR rows of nch partials.  The new state in shared memory; false: finished.
+  __device__ __forceinline__ bool run(const Seg &S, int chunk, int inst, const double *__restrict__ part,
+                                      const KState *__restrict__ in, KState *__restrict__ out, KState &ks) {
+    constexpr int WORDS = sizeof(KState) / 4;
+    __shared__ double red[NR][BB / 64];
+    const bool first = chunk == S.ch_first[inst];
+    const int c0 = S.ch_first[inst], c1 = S.ch_first[inst + 1];
+    uint32_t word = 0;
+    if (threadIdx.x < WORDS) word = reinterpret_cast<const uint32_t *>(in + inst)[threadIdx.x];
+#pragma unroll
+    for (int q = 0; q < NR; q++) a[q] = 0.0;
+    for (int c = c0 + threadIdx.x; c < c1; c += BB)
+#pragma unroll
+      for (int q = 0; q < NR; q++) a[q] += part[(size_t)q * S.nch + c];
+    if (threadIdx.x < WORDS) reinterpret_cast<uint32_t *>(&ks)[threadIdx.x] = word;
+#pragma unroll
+    for (int q = 0; q < NR; q++) {
+      a[q] = wave_sum(a[q]);
+      if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = a[q];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && !ks.done) {
+      double tot[NR];
+#pragma unroll
+      for (int q = 0; q < NR; q++) tot[q] = (red[q][0] + red[q][1]) + (red[q][2] + red[q][3]);
+      if (STAGE == STAGE_XR && ks.pad)
+        ks.pad = 0;
+      else
+        run_stage<STAGE>(&ks, tot);
+    }
+    __syncthreads();
+    if (first && threadIdx.x < WORDS)
+      reinterpret_cast<uint32_t *>(out + inst)[threadIdx.x] = reinterpret_cast<const uint32_t *>(&ks)[threadIdx.x];
+    return !ks.done;
+  }
+};
+
+template <int NR>
+__device__ __forceinline__ void chunk_partials(const Seg &S, int chunk, const double (&v)[NR], double *__restrict__ part) {
+  __shared__ double red[NR][BB / 64];
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    const double w = wave_sum(v[q]);
+    if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = w;
+  }
+  __syncthreads();
+  if (threadIdx.x < NR)
+    part[(size_t)threadIdx.x * S.nch + chunk] = (red[threadIdx.x][0] + red[threadIdx.x][1]) +
+                                                     (red[threadIdx.x][2] + red[threadIdx.x][3]);
+}
+
+// states and partial sums of the form above
+struct BKry {
+  KState *st, *s1, *s2;
+  double *rho, *alpha, *omega;  // 2, 1 and 3 rows of nch
+};
+
 template <class V>
 __device__ __forceinline__ V bicg_s(V r, V v, double alpha) {
   return (V)__builtin_fma(-alpha, (double)v, (double)r);
 }
+template <class V>
+__device__ __forceinline__ V bicg_p(V r, V p, V v, double beta, double omega) {
+  return (V)((double)r + beta * ((double)p - omega * (double)v));
+}
 
-template <class VA, class V, bool NT, class CI>
-__global__ void __launch_bounds__(BB) k_bspmv_s(Seg S, const int32_t *__restrict__ ch_slice,
-                                                const int32_t *__restrict__ sptr, const CI *__restrict__ col,
-                                                const VA *__restrict__ val, const V *__restrict__ r,
-                                                const V *__restrict__ v, V *__restrict__ s, V *__restrict__ t,
-                                                KState *st, unsigned long long *__restrict__ mwork,
-                                                const int64_t *__restrict__ msize) {
-  const int inst = S.ch_inst[blockIdx.x];
-  const KState *sti = st + inst;
-  if (sti->done) return;
-  const double alpha = sti->alpha;
-  const int64_t r0 = S.ch_beg[blockIdx.x], r1 = S.ch_end[blockIdx.x];
-  if (mwork && threadIdx.x == 0 && blockIdx.x == S.ch_first[inst]) {  // probe counters, as k_bspmv
+// row l of the chunk times y(column)
+template <class VA, bool NT, class CI, class F>
+__device__ __forceinline__ double chunk_row(int64_t row, int32_t sl, int l, const int32_t *__restrict__ sptr,
+                                            const CI *__restrict__ col, const VA *__restrict__ val, F &&y) {
+  const int32_t p1 = sptr[sl + 1];
+  double acc = 0.0;
+#pragma unroll 4
+  for (int32_t q = sptr[sl] + l; q < p1; q += 64)
+    acc += (double)bld<NT>(val + q) * (double)y(sell_column(bld<NT>(col + q), row));
+  return acc;
+}
+
+// probe counters, as k_bspmv
+__device__ __forceinline__ void count_member(const Seg &S, int chunk, int inst, unsigned long long *mwork,
+                                             const int64_t *__restrict__ msize) {
+  if (mwork && threadIdx.x == 0 && chunk == S.ch_first[inst]) {
     mwork[2 * inst] += (unsigned long long)msize[2 * inst];
     mwork[2 * inst + 1] += (unsigned long long)msize[2 * inst + 1];
   }
-  const int32_t sl0 = ch_slice[blockIdx.x];
+}
+
+// last update's sums, p' and v' = Ahat p'; partials of (r0, v')
+template <class VA, class V, bool NT, class CI>
+__global__ void __launch_bounds__(BB) k_bpv(Seg S, const int32_t *__restrict__ ch_slice,
+                                            const int32_t *__restrict__ sptr, const CI *__restrict__ col,
+                                            const VA *__restrict__ val, const V *__restrict__ r,
+                                            const V *__restrict__ p, const V *__restrict__ v, V *__restrict__ pn,
+                                            V *__restrict__ vn, const V *__restrict__ r0, BKry K,
+                                            unsigned long long *__restrict__ mwork,
+                                            const int64_t *__restrict__ msize) {
+  const int c = chunk_of(S);
+  if (c < 0) return;
+  const int inst = S.ch_inst[c];
+  __shared__ KState ks;
+  BFold<STAGE_XR, 2> f;
+  if (!f.run(S, c, inst, K.rho, K.st, K.s1, ks)) return;
+  count_member(S, c, inst, mwork, msize);
+  const double beta = ks.beta, omega = ks.omega;
+  const int64_t i0 = S.ch_beg[c], i1 = S.ch_end[c];
+  const int32_t sl0 = ch_slice[c];
+  double d = 0.0;
+  for (int64_t l = threadIdx.x; l < i1 - i0; l += BB) {
+    const int64_t i = i0 + l;
+    const V vv = (V)chunk_row<VA, NT, CI>(i, sl0 + (int32_t)(l >> 6), (int)(l & 63), sptr, col, val,
+                                          [&](int64_t j) { return bicg_p(r[j], p[j], v[j], beta, omega); });
+    pn[i] = bicg_p(r[i], p[i], v[i], beta, omega);
+    vn[i] = vv;
+    d += (double)r0[i] * (double)vv;
+  }
+  double dd[1] = {d};
+  chunk_partials<1>(S, c, dd, K.alpha);
+}
+
+// alpha, t = Ahat s with s = r - alpha v; partials of (s, t), (t, t), (s, s)
+template <class VA, class V, bool NT, class CI>
+__global__ void __launch_bounds__(BB) k_bst(Seg S, const int32_t *__restrict__ ch_slice,
+                                            const int32_t *__restrict__ sptr, const CI *__restrict__ col,
+                                            const VA *__restrict__ val, const V *__restrict__ r,
+                                            const V *__restrict__ v, V *__restrict__ t, BKry K,
+                                            unsigned long long *__restrict__ mwork,
+                                            const int64_t *__restrict__ msize) {
+  const int c = chunk_of(S);
+  if (c < 0) return;
+  const int inst = S.ch_inst[c];
+  __shared__ KState ks;
+  BFold<STAGE_ALPHA, 1> f;
+  if (!f.run(S, c, inst, K.alpha, K.s1, K.s2, ks)) return;
+  count_member(S, c, inst, mwork, msize);
+  const double alpha = ks.alpha;
+  const int64_t i0 = S.ch_beg[c], i1 = S.ch_end[c];
+  const int32_t sl0 = ch_slice[c];
   double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-  for (int64_t l = threadIdx.x; l < r1 - r0; l += BB) {
-    const int32_t sl = sl0 + (int32_t)(l >> 6);
-    const int32_t p1 = sptr[sl + 1];
-    const int64_t row = r0 + l;
-    double acc = 0.0;
-#pragma unroll 4
-    for (int32_t q = sptr[sl] + (int32_t)(l & 63); q < p1; q += 64) {
-      const int64_t j = sell_column(bld<NT>(col + q), row);
-      acc += (double)bld<NT>(val + q) * (double)bicg_s(r[j], v[j], alpha);
-    }
-    const V tv = (V)acc;
-    const V sv = bicg_s(r[row], v[row], alpha);
-    t[row] = tv;
-    s[row] = sv;
+  for (int64_t l = threadIdx.x; l < i1 - i0; l += BB) {
+    const int64_t i = i0 + l;
+    const V tv = (V)chunk_row<VA, NT, CI>(i, sl0 + (int32_t)(l >> 6), (int)(l & 63), sptr, col, val,
+                                          [&](int64_t j) { return bicg_s(r[j], v[j], alpha); });
+    const V sv = bicg_s(r[i], v[i], alpha);
+    t[i] = tv;
     d0 += (double)sv * (double)tv;
     d1 += (double)tv * (double)tv;
     d2 += (double)sv * (double)sv;
   }
-  double vv[3] = {d0, d1, d2};
-  seg_partials<3, false>(S, vv, 0.0);
+  double dd[3] = {d0, d1, d2};
+  chunk_partials<3>(S, c, dd, K.omega);
+}
+
+// half-step test and omega; x += alpha p + omega s, r = s - omega t; partials of (r0, r), (r, r)
+template <class V>
+__global__ void __launch_bounds__(BB) k_bxr3(Seg S, V *__restrict__ x, const V *__restrict__ p,
+                                             const V *__restrict__ v, const V *__restrict__ t, V *__restrict__ r,
+                                             const V *__restrict__ r0, BKry K) {
+  const int c = chunk_of(S);
+  if (c < 0) return;
+  const int inst = S.ch_inst[c];
+  __shared__ KState ks;
+  BFold<STAGE_SOMEGA, 3> f;
+  if (!f.run(S, c, inst, K.omega, K.s2, K.st, ks)) return;
+  const double alpha = ks.alpha, omega = ks.omega;
+  const bool half = ks.half != 0;
+  double d0 = 0.0, d1 = 0.0;
+  const int64_t i1 = S.ch_end[c];
+  for (int64_t i = S.ch_beg[c] + threadIdx.x; i < i1; i += BB) {
+    if (half) {
+      x[i] = (V)((double)x[i] + alpha * (double)p[i]);
+    } else {
+      const V sv = bicg_s(r[i], v[i], alpha);
+      x[i] = (V)((double)x[i] + alpha * (double)p[i] + omega * (double)sv);
+      const V rv = (V)((double)sv - omega * (double)t[i]);
+      r[i] = rv;
+      d0 += (double)r0[i] * (double)rv;
+      d1 += (double)rv * (double)rv;
+    }
+  }
+  double dd[2] = {d0, d1};
+  chunk_partials<2>(S, c, dd, K.rho);
+}
+
+// the states after the last queued iteration, to pinned host memory (one block per member)
+__global__ void __launch_bounds__(BB) k_breport(Seg S, BKry K, KState *__restrict__ pinned) {
+  const int m = blockIdx.x;
+  __shared__ KState ks;
+  __shared__ double sh[16];
+  if (threadIdx.x == 0) ks = K.st[m];
+  double a[2] = {0.0, 0.0};
+  for (int c = S.ch_first[m] + threadIdx.x; c < S.ch_first[m + 1]; c += BB)
+    for (int q = 0; q < 2; q++) a[q] += K.rho[(size_t)q * S.nch + c];
+  for (int q = 0; q < 2; q++) a[q] = bsum(a[q], sh);
+  if (threadIdx.x != 0) return;
+  if (!ks.done && !ks.pad) run_stage<STAGE_XR>(&ks, a);
+  pinned[m] = ks;
 }
 
 // y = S (b - A x), ||y||^2 per member -> st.rr (FP64; refinement residual and bhat)
@@ -638,7 +814,12 @@ struct vfvm_batch {
   int64_t sell_nnz = 0;
   // probe work of the batched SpMV: per member (rows, nonzeros) and per-member counters
   DevBuf<int64_t> msize;
-  DevBuf<unsigned long long> mwork, mwork_half;  // k_bspmv's and k_bspmv_s's counters
+  DevBuf<unsigned long long> mwork, mwork_half;  // the counters of k_bspmv and k_bpv, and of k_bst
+  DevBuf<KState> st1, st2;  // point Jacobi BiCGStab, one launch per Krylov step (BKry)
+  DevBuf<double> kpart;
+  BKry kry() const {
+    return {st.p, st1.p, st2.p, kpart.p, kpart.p + 2 * nch, kpart.p + 3 * nch};
+  }
   bool sell_nt[2] = {false, false};  // non-temporal matrix loads in the SpMV (FP32, FP64)
   // captured Krylov iteration blocks: (value bytes, solution vector, iterations) -> graph
   bool use_graphs = true;
@@ -766,26 +947,37 @@ void bop(vfvm_batch &b, const V *x, V *y, const V *w0) {
                        b.st.p, (const int32_t *)nullptr, (double *)nullptr);
 }
 
-// s = r - alpha v, t = Ahat s, and STAGE_SOMEGA (see k_bspmv_s)
+// one point Jacobi BiCGStab iteration (k_bpv and the kernels after it); p, v and pn, vn change roles
 template <class V>
-void bop_s(vfvm_batch &b, const V *r, const V *v, V *s, V *t) {
+void bstep(vfvm_batch &b, V *x, V *r, const V *r0, const V *p, const V *v, V *pn, V *vn, V *t) {
   const Seg S = b.seg();
-  const int kid = sizeof(V) == 4 ? VFVM_KERNEL_HALFSTEP32 : VFVM_KERNEL_HALFSTEP64;
-  unsigned long long *mwork = b.ctx->probe.counters(kid) ? b.mwork_half.p : nullptr;
-  b.ctx->probe.before(kid, b.ctx->stream);
+  const BKry K = b.kry();
+  hipStream_t st = b.ctx->stream;
+  const V *val;
+  if constexpr (sizeof(V) == 4) val = b.A32.p;
+  else val = b.A64s.p;
+  const int64_t *msize = b.msize.p;
   auto go = [&](auto ntc, const auto *col) {
     constexpr bool NT = decltype(ntc)::value;
     using CI = std::remove_const_t<std::remove_pointer_t<decltype(col)>>;
-    if constexpr (sizeof(V) == 4)
-      VFVM_LAUNCH((k_bspmv_s<float, V, NT, CI>), dim3((unsigned)b.nch), dim3(BB), 0, b.ctx->stream, S,
-                  (const int32_t *)b.ch_slice.p, (const int32_t *)b.sell_ptr.p, col, (const float *)b.A32.p, r, v, s,
-                  t, b.st.p, mwork, (const int64_t *)b.msize.p);
-    else
-      VFVM_LAUNCH((k_bspmv_s<double, V, NT, CI>), dim3((unsigned)b.nch), dim3(BB), 0, b.ctx->stream, S,
-                  (const int32_t *)b.ch_slice.p, (const int32_t *)b.sell_ptr.p, col, (const double *)b.A64s.p, r, v,
-                  s, t, b.st.p, mwork, (const int64_t *)b.msize.p);
+    const int ks = sizeof(V) == 4 ? VFVM_KERNEL_SPMV32 : VFVM_KERNEL_SPMV64;
+    b.ctx->probe.before(ks, st);
+    VFVM_LAUNCH((k_bpv<V, V, NT, CI>), dim3(chunk_grid(b.nch)), dim3(BB), 0, st, S, (const int32_t *)b.ch_slice.p,
+                (const int32_t *)b.sell_ptr.p, col, val, (const V *)r, p, v, pn, vn, r0, K,
+                b.ctx->probe.counters(ks) ? b.mwork.p : nullptr, msize);
+    b.ctx->probe.after(ks, st);
+    const int kh = sizeof(V) == 4 ? VFVM_KERNEL_HALFSTEP32 : VFVM_KERNEL_HALFSTEP64;
+    b.ctx->probe.before(kh, st);
+    VFVM_LAUNCH((k_bst<V, V, NT, CI>), dim3(chunk_grid(b.nch)), dim3(BB), 0, st, S, (const int32_t *)b.ch_slice.p,
+                (const int32_t *)b.sell_ptr.p, col, val, (const V *)r, (const V *)vn, t, K,
+                b.ctx->probe.counters(kh) ? b.mwork_half.p : nullptr, msize);
+    b.ctx->probe.after(kh, st);
   };
-  const bool nt = b.sell_nt[sizeof(V) == 4 ? 0 : 1];
+  // Non-temporal matrix loads only for a matrix that the caches do not hold between products: a solve
+  // takes, with them and without, 79 and 69 ms for 64 uneven members (60 MB), 27 and 24 ms for 256 of
+  // 65^2 rows (54 MB), 193 and 196 ms for 512 of 129^2 in FP32 (255 MB), 261 and 268 ms in FP64.
+  const size_t bytes = (sizeof(V) == 4 ? b.A32.n * 4 : b.A64s.n * 8) / sizeof(V) * (sizeof(V) + 2);
+  const bool nt = b.sell_nt[sizeof(V) == 4 ? 0 : 1] && bytes > (size_t)128 << 20;
   if (b.sell_off16.p && b.sell16) {
     if (nt)
       go(std::true_type(), (const int16_t *)b.sell_off16.p);
@@ -797,9 +989,8 @@ void bop_s(vfvm_batch &b, const V *r, const V *v, V *s, V *t) {
     else
       go(std::false_type(), (const int32_t *)b.sell_col.p);
   }
-  b.ctx->probe.after(kid, b.ctx->stream);
-  hipLaunchKernelGGL((k_bfinalize<3, STAGE_SOMEGA, BF_STAGE>), dim3((unsigned)b.nsys), dim3(BB), 0, b.ctx->stream, S,
-                     b.st.p, (const int32_t *)nullptr, (double *)nullptr);
+  hipLaunchKernelGGL((k_bxr3<V>), dim3(chunk_grid(b.nch)), dim3(BB), 0, st, S, x, (const V *)pn, (const V *)vn,
+                     (const V *)t, r, r0, K);
 }
 
 void bres(vfvm_batch &b, const double *x, const double *rhs, double *y, const int32_t *active) {
@@ -926,7 +1117,21 @@ int bbicgstab(vfvm_batch &b, const VBin *bh, V *x, const int32_t *active, double
       ph = b.kp64[0].p; sh = b.kp64[1].p;
     }
   }
-  if (amg) b.amg.reserve<V>();
+  if (amg) {
+    b.amg.reserve<V>();
+  } else if (!b.member_bs) {
+    V *&second = ph;  // v of every other iteration
+    if constexpr (sizeof(V) == 4) {
+      b.kp32[0].alloc((size_t)b.ndof);
+      second = b.kp32[0].p;
+    } else {
+      b.kp64[0].alloc((size_t)b.ndof);
+      second = b.kp64[0].p;
+    }
+    b.st1.alloc((size_t)b.nsys);
+    b.st2.alloc((size_t)b.nsys);
+    b.kpart.alloc((size_t)6 * b.nch);
+  }
   reset_states(b, rtol, atol, maxit);
   if (b.member_bs) {
     msolve<V>(b, bh, x, r, r0, p, v, s, t, ph, sh, active, amg);
@@ -946,7 +1151,8 @@ int bbicgstab(vfvm_batch &b, const VBin *bh, V *x, const int32_t *active, double
   hipLaunchKernelGGL((k_binit<V, VBin>), dim3((unsigned)b.nch), dim3(BB), 0, st, S, bh, r, r0, p, v, x, b.st.p, active);
   hipLaunchKernelGGL((k_bfinalize<1, STAGE_INIT, BF_INIT>), dim3((unsigned)b.nsys), dim3(BB), 0, st, S, b.st.p, active,
                      (double *)nullptr);
-  const int every = std::max(1, check_every);
+  // point Jacobi: a pair of iterations leaves p and v where they were (the block may be a graph)
+  const int every = amg ? std::max(1, check_every) : (std::max(1, check_every) + 1) / 2 * 2;
   int launched = 0;
   std::vector<KState> h;
   // `every` iterations between status reads; kernels of finished members return at entry
@@ -966,12 +1172,9 @@ int bbicgstab(vfvm_batch &b, const VBin *bh, V *x, const int32_t *active, double
                            b.st.p, (const int32_t *)nullptr, (double *)nullptr);
         continue;
       }
-      hipLaunchKernelGGL((k_bp<V>), dim3((unsigned)b.nch), dim3(BB), 0, st, S, r, p, v, b.st.p);
-      bop<V, 1, STAGE_ALPHA>(b, p, v, r0);
-      bop_s<V>(b, r, v, s, t);  // s = r - alpha v, t = Ahat s, half-step test and omega
-      hipLaunchKernelGGL((k_bxr<V>), dim3((unsigned)b.nch), dim3(BB), 0, st, S, x, p, s, s, t, r, r0, b.st.p);
-      hipLaunchKernelGGL((k_bfinalize<2, STAGE_XR, BF_STAGE>), dim3((unsigned)b.nsys), dim3(BB), 0, st, S, b.st.p,
-                         (const int32_t *)nullptr, (double *)nullptr);
+      bstep<V>(b, x, r, r0, p, v, s, ph, t);
+      std::swap(p, s);
+      std::swap(v, ph);
     }
   };
   // The block is captured once into a HIP graph (its kernel arguments are fixed for the
@@ -998,8 +1201,7 @@ int bbicgstab(vfvm_batch &b, const VBin *bh, V *x, const int32_t *active, double
   // Pipelined: the next block of `every` iterations is queued before the states after
   // the current block are examined, so the device never waits for the host's decision.
   // A block queued after every member has finished only runs kernels that return at
-  // entry.  Each block ends with an asynchronous copy of the states into its own pinned
-  // slot.
+  // entry.  Each block ends with the states' way into its own pinned slot.
   auto enqueue = [&](int slot) {
     if (ge)
       VFVM_HIP_CHECK(hipGraphLaunch(ge, st));
@@ -1007,7 +1209,10 @@ int bbicgstab(vfvm_batch &b, const VBin *bh, V *x, const int32_t *active, double
       body();
     VFVM_HIP_CHECK(hipGetLastError());
     launched += every;
-    VFVM_HIP_CHECK(hipMemcpyAsync(b.hst[slot], b.st.p, sizeof(KState) * b.nsys, hipMemcpyDeviceToHost, st));
+    if (amg)
+      VFVM_HIP_CHECK(hipMemcpyAsync(b.hst[slot], b.st.p, sizeof(KState) * b.nsys, hipMemcpyDeviceToHost, st));
+    else
+      hipLaunchKernelGGL(k_breport, dim3((unsigned)b.nsys), dim3(BB), 0, st, S, b.kry(), b.hst[slot]);
     VFVM_HIP_CHECK(hipEventRecord(b.sev[slot], st));
   };
   int slot = 0, last = 0;

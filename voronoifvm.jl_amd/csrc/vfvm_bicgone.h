@@ -23,12 +23,7 @@ __device__ __forceinline__ void one_sum(double (&v)[NR], double (*red)[3][ONE_T 
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NR; k++) {
-    double w = rb[k][threadIdx.x & 15];
-    w = add_dpp<0xB1>(w);
-    w = add_dpp<0x4E>(w);
-    w = add_dpp<0x141>(w);
-    w = add_dpp<0x140>(w);
-    v[k] = lane_value(w, 0);
+    v[k] = lane_value(row_sum(rb[k][threadIdx.x & 15]), 0);
   }
 }
 
