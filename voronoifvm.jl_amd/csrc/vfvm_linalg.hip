@@ -1086,9 +1086,11 @@ int LinearSolver::bicgstab(const VBin *b, VXo *x, const double *J, const vfvm_co
   }
   VFVM_HIP_CHECK(hipMemcpyAsync(st.p, &h, sizeof(KState), hipMemcpyHostToDevice, stream));
   K.init(b);
-  // first chunk: about as many iterations as the previous solve needed (Newton steps of one
-  // solve need similar counts), then poll every check_every iterations
-  const int every = std::max(1, c.check_every);
+  // First chunk: about as many iterations as the previous solve needed (Newton steps of one
+  // solve need similar counts), then poll every check_every iterations; an iteration with
+  // multigrid costs more than a poll (40 launches even when it has nothing left to do), so
+  // there every one: of 123 iterations queued in a Newton solve on 513^2 rows 72 were needed.
+  const int every = c.precon == VFVM_PRECON_AMG ? 1 : std::max(1, c.check_every);
   int check = std::max(every, std::min(maxit, last_iters - 1));
   int launched = 0, best_at = 0;
   double best = -1.0;
