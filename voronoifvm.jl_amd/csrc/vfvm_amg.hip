@@ -270,10 +270,14 @@ struct SView {
   const int32_t *idx;
   const V *val;
 };
-// one slice per wave and one entry per round: the form that measured fastest (more
-// slices or entries per wave raise the registers and cut occupancy by more than they gain)
-constexpr int SPW = 1;     // slices per wave
-constexpr int UNROLL = 1;  // row entries per round of loads
+// One slice per wave (more raise the registers and cut occupancy by more than they gain).
+constexpr int SPW = 1;  // slices per wave
+// Row entries per round of loads.  Up to FEW_SLICES slices (8 waves a SIMD at most) no other waves
+// hide the latency of an entry's two dependent loads, which a row pays once per round: on 513^2 rows
+// (4,112 slices on the finest level) restriction, residual, sweep and prolongation take 13.3, 8.9,
+// 5.7 and 4.4 us a level with 1 entry a round, 6.0, 6.1, 4.1 and 3.6 with 4, 4.7, 5.6, 3.8 and 3.9
+// with 8.  More slices keep 1 (more registers cost occupancy).
+constexpr int FEW_SLICES = 8192, FEW_UNROLL = 8;
 
 struct Lane {
   SellDesc d;
@@ -303,39 +307,41 @@ __device__ __forceinline__ bool amg_lanes(const SView<VA> &M, const int32_t *mod
   return any;
 }
 
-// acc[k] = sum_j M[row_k, j] f(k, column) for the wave's rows
-template <class V, class F>
+// acc[k] = sum_j M[row_k, j] f(k, column) for the wave's rows.  A round's loads have no conditions
+// of their own (past the row's width they repeat its last entry, which is not added): with a
+// condition each the compiler waits for one before the next.
+template <int UNROLL, class V, class F>
 __device__ __forceinline__ void amg_rows(const SView<V> &M, const Lane (&L)[SPW], F &&f, double (&acc)[SPW]) {
   const int lane = threadIdx.x & 63;
-  int32_t w = 0;
 #pragma unroll
   for (int k = 0; k < SPW; k++) {
     acc[k] = 0.0;
-    if (L[k].on) w = max(w, L[k].d.width);
-  }
-  for (int32_t j0 = 0; j0 < w; j0 += UNROLL) {
-    int32_t c[SPW][UNROLL];
-    V a[SPW][UNROLL];
-#pragma unroll
-    for (int k = 0; k < SPW; k++)
+    if (!L[k].on) continue;
+    const int32_t w = __builtin_amdgcn_readfirstlane(L[k].d.width);
+    const int32_t *ip = M.idx + (int64_t)L[k].d.ibase + lane;
+    const V *vp = M.val + L[k].d.vbase + lane;
+    for (int32_t j0 = 0; j0 < w; j0 += UNROLL) {
+      int32_t c[UNROLL];
+      V a[UNROLL];
+      double y[UNROLL];
 #pragma unroll
       for (int u = 0; u < UNROLL; u++) {
-        const bool ok = L[k].on && j0 + u < L[k].d.width;
-        const int64_t off = (int64_t)lane + (int64_t)64 * (j0 + u);
-        c[k][u] = ok ? M.idx[(int64_t)L[k].d.ibase + off] : 0;
-        a[k][u] = ok ? M.val[L[k].d.vbase + off] : (V)0;
+        const int32_t j = UNROLL == 1 ? j0 : min(j0 + u, w - 1);
+        c[u] = ip[64 * j];
+        a[u] = vp[64 * j];
       }
 #pragma unroll
-    for (int k = 0; k < SPW; k++)
+      for (int u = 0; u < UNROLL; u++) y[u] = f(k, (int64_t)L[k].d.coff + c[u]);
 #pragma unroll
       for (int u = 0; u < UNROLL; u++)
-        if (L[k].on && j0 + u < L[k].d.width) acc[k] += (double)a[k][u] * f(k, (int64_t)L[k].d.coff + c[k][u]);
+        if (UNROLL == 1 || j0 + u < w) acc[k] += (double)a[u] * y[u];
+    }
   }
 }
 
 // pre-smoothing from zero and the residual on the rows of coarsening members:
 // r = b - A x with x = omega D^-1 b (x itself is not stored: the prolongation recomputes it)
-template <class V>
+template <class V, int UNROLL>
 __global__ void __launch_bounds__(AB) k_amg_down(SView<AmgVal<V>> A, const V *__restrict__ dinv,
                                                  const double *__restrict__ w, const int32_t *__restrict__ mode,
                                                  const V *__restrict__ b, V *__restrict__ r, const KState *st,
@@ -345,27 +351,27 @@ __global__ void __launch_bounds__(AB) k_amg_down(SView<AmgVal<V>> A, const V *__
   double wm[SPW], acc[SPW];
 #pragma unroll
   for (int k = 0; k < SPW; k++) wm[k] = L[k].on ? w[L[k].d.inst] : 0.0;
-  amg_rows(A, L, [&](int k, int64_t c) { return wm[k] * (dinv ? (double)dinv[c] : 1.0) * (double)b[c]; }, acc);
+  amg_rows<UNROLL>(A, L, [&](int k, int64_t c) { return wm[k] * (dinv ? (double)dinv[c] : 1.0) * (double)b[c]; }, acc);
 #pragma unroll
   for (int k = 0; k < SPW; k++)
     if (L[k].on) r[L[k].row] = (V)((double)b[L[k].row] - acc[k]);
 }
 
 // b_coarse = P^T r (every row of the next level belongs to a coarsening member)
-template <class V>
+template <class V, int UNROLL>
 __global__ void __launch_bounds__(AB) k_amg_restrict(SView<AmgVal<V>> R, const V *__restrict__ r,
                                                      V *__restrict__ bc, const KState *st, int skip_half) {
   Lane L[SPW];
   if (!amg_lanes(R, (const int32_t *)nullptr, 0, st, skip_half, L)) return;
   double acc[SPW];
-  amg_rows(R, L, [&](int, int64_t c) { return (double)r[c]; }, acc);
+  amg_rows<UNROLL>(R, L, [&](int, int64_t c) { return (double)r[c]; }, acc);
 #pragma unroll
   for (int k = 0; k < SPW; k++)
     if (L[k].on) bc[L[k].row] = (V)acc[k];
 }
 
 // x = omega D^-1 b + P x_coarse on the rows of coarsening members
-template <class V>
+template <class V, int UNROLL>
 __global__ void __launch_bounds__(AB) k_amg_prolong(SView<AmgVal<V>> P, const V *__restrict__ dinv,
                                                     const double *__restrict__ w, const int32_t *__restrict__ mode,
                                                     const V *__restrict__ b, const V *__restrict__ xc,
@@ -373,7 +379,7 @@ __global__ void __launch_bounds__(AB) k_amg_prolong(SView<AmgVal<V>> P, const V 
   Lane L[SPW];
   if (!amg_lanes(P, mode, Amg::MODE_COARSEN, st, skip_half, L)) return;
   double acc[SPW];
-  amg_rows(P, L, [&](int, int64_t c) { return (double)xc[c]; }, acc);
+  amg_rows<UNROLL>(P, L, [&](int, int64_t c) { return (double)xc[c]; }, acc);
 #pragma unroll
   for (int k = 0; k < SPW; k++)
     if (L[k].on) {
@@ -386,7 +392,7 @@ __global__ void __launch_bounds__(AB) k_amg_prolong(SView<AmgVal<V>> P, const V 
 // mode (post-smoothing of coarsening members, sweeps on a large coarsest level).  dwork
 // (probe counters, nullable): the first slice of each member it runs on adds the member's
 // rows and nonzeros (msize), one atomic pair per member and launch.
-template <class V>
+template <class V, int UNROLL>
 __global__ void __launch_bounds__(AB) k_amg_sweep(SView<AmgVal<V>> A, const V *__restrict__ dinv,
                                                   const double *__restrict__ w, const int32_t *__restrict__ mode,
                                                   int want, const V *__restrict__ b, const V *__restrict__ x,
@@ -395,7 +401,7 @@ __global__ void __launch_bounds__(AB) k_amg_sweep(SView<AmgVal<V>> A, const V *_
   Lane L[SPW];
   if (!amg_lanes(A, mode, want, st, skip_half, L)) return;
   double acc[SPW];
-  amg_rows(A, L, [&](int, int64_t c) { return (double)x[c]; }, acc);
+  amg_rows<UNROLL>(A, L, [&](int, int64_t c) { return (double)x[c]; }, acc);
 #pragma unroll
   for (int k = 0; k < SPW; k++) {
     if (!L[k].on) continue;
@@ -1279,6 +1285,12 @@ void Amg::apply(const V *y, V *z, const KState *st, int skip_half, hipStream_t s
     if constexpr (F32) return L.dinvA32.p;
     else return L.dinvA64.p;
   };
+  auto by_waves = [](int64_t nsl, auto &&launch) {
+    if (nsl <= FEW_SLICES)
+      launch(std::integral_constant<int, FEW_UNROLL>());
+    else
+      launch(std::integral_constant<int, 1>());
+  };
   auto grid = [](const SellMat &M) {
     const int64_t per_block = (AB / 64) * SPW;
     return (unsigned)std::max<int64_t>(1, (M.nsl + per_block - 1) / per_block);
@@ -1288,10 +1300,14 @@ void Amg::apply(const V *y, V *z, const KState *st, int skip_half, hipStream_t s
     Lev &L = lev[l];
     const SView<AmgVal<V>> A = view(L.A);
     if (L.any_coarsen) {
-      hipLaunchKernelGGL((k_amg_down<V>), dim3(grid(L.A)), dim3(AB), 0, s, A, dinv(l), (const double *)L.w.p,
-                         (const int32_t *)L.mode.p, bof(l), R[l], st, skip_half);
-      hipLaunchKernelGGL((k_amg_restrict<V>), dim3(grid(L.R)), dim3(AB), 0, s, view(L.R), (const V *)R[l],
-                         B[l + 1], st, skip_half);
+      by_waves(A.nsl, [&](auto u) {
+        hipLaunchKernelGGL((k_amg_down<V, decltype(u)::value>), dim3(grid(L.A)), dim3(AB), 0, s, A, dinv(l),
+                           (const double *)L.w.p, (const int32_t *)L.mode.p, bof(l), R[l], st, skip_half);
+      });
+      by_waves(L.R.nsl, [&](auto u) {
+        hipLaunchKernelGGL((k_amg_restrict<V, decltype(u)::value>), dim3(grid(L.R)), dim3(AB), 0, s, view(L.R),
+                           (const V *)R[l], B[l + 1], st, skip_half);
+      });
     }
     if (L.ndm)
       hipLaunchKernelGGL((k_amg_dense_apply<V>), dim3((unsigned)L.ndm), dim3(AB), 0, s, (const int32_t *)L.dmem.p,
@@ -1302,9 +1318,11 @@ void Amg::apply(const V *y, V *z, const KState *st, int skip_half, hipStream_t s
                          (const int32_t *)L.mode.p, bof(l), X[l], st, skip_half);
       V *a = X[l], *o = sol(l);
       for (int k = 1; k < COARSE_SWEEPS; k++) {  // an odd count of sweeps ends in sol(l)
-        hipLaunchKernelGGL((k_amg_sweep<V>), dim3(grid(L.A)), dim3(AB), 0, s, A, dinv(l), (const double *)L.w.p,
-                           (const int32_t *)L.mode.p, (int)MODE_JACOBI, bof(l), (const V *)a, o, st, skip_half,
-                           (unsigned long long *)nullptr, (const int64_t *)nullptr);
+        by_waves(A.nsl, [&](auto u) {
+          hipLaunchKernelGGL((k_amg_sweep<V, decltype(u)::value>), dim3(grid(L.A)), dim3(AB), 0, s, A, dinv(l),
+                             (const double *)L.w.p, (const int32_t *)L.mode.p, (int)MODE_JACOBI, bof(l), (const V *)a,
+                             o, st, skip_half, (unsigned long long *)nullptr, (const int64_t *)nullptr);
+        });
         std::swap(a, o);
       }
     }
@@ -1320,14 +1338,20 @@ void Amg::apply(const V *y, V *z, const KState *st, int skip_half, hipStream_t s
   for (int l = std::min(nlev, lt) - 1; l >= 0; l--) {
     Lev &L = lev[l];
     if (!L.any_coarsen) continue;
-    hipLaunchKernelGGL((k_amg_prolong<V>), dim3(grid(L.P)), dim3(AB), 0, s, view(L.P), dinv(l), (const double *)L.w.p,
-                       (const int32_t *)L.mode.p, bof(l), (const V *)sol(l + 1), X[l], st, skip_half);
+    by_waves(L.P.nsl, [&](auto u) {
+      hipLaunchKernelGGL((k_amg_prolong<V, decltype(u)::value>), dim3(grid(L.P)), dim3(AB), 0, s, view(L.P), dinv(l),
+                         (const double *)L.w.p, (const int32_t *)L.mode.p, bof(l), (const V *)sol(l + 1), X[l], st,
+                         skip_half);
+    });
     const int kid = F32 ? VFVM_KERNEL_AMG32 : VFVM_KERNEL_AMG64;
     const bool probed = l == 0 && probe && probe->counters(kid);
     if (probed) probe->before(kid, s);
-    VFVM_LAUNCH((k_amg_sweep<V>), dim3(grid(L.A)), dim3(AB), 0, s, view(L.A), dinv(l), (const double *)L.w.p,
-                (const int32_t *)L.mode.p, (int)MODE_COARSEN, bof(l), (const V *)X[l], sol(l), st, skip_half,
-                probed ? probe->counters(kid) : (unsigned long long *)nullptr, (const int64_t *)msize0.p);
+    by_waves(L.A.nsl, [&](auto u) {
+      VFVM_LAUNCH((k_amg_sweep<V, decltype(u)::value>), dim3(grid(L.A)), dim3(AB), 0, s, view(L.A), dinv(l),
+                  (const double *)L.w.p, (const int32_t *)L.mode.p, (int)MODE_COARSEN, bof(l), (const V *)X[l], sol(l),
+                  st, skip_half, probed ? probe->counters(kid) : (unsigned long long *)nullptr,
+                  (const int64_t *)msize0.p);
+    });
     if (probed) probe->after(kid, s);
   }
 }
