@@ -75,11 +75,12 @@ __device__ __forceinline__ MemberMat<VA> member_mat(const SellDesc *d, const int
   return M;
 }
 
-// sum_j M[row, j] f(column) for the lane's row of slice d: the index and value loads of
-// the first W entries are issued together (positions past the slice's width re-read its
-// last entry, so every address is valid and no branch splits the loads), then their
-// gathers, so a row costs about two memory round trips instead of two per entry; wider
-// rows finish in a loop
+// sum_j M[row, j] f(column) for the lane's row of slice d: the index and value loads of W
+// entries are issued together (positions past the slice's width re-read its last entry,
+// so every address is valid and no branch splits the loads), then their gathers, so a row
+// costs about two memory round trips per W entries instead of two per entry
+// (with only the first W taken so, the restriction rows of 10 to 20 entries finished one by one:
+// 5.37 ms a launch of k_msolve for 512 members of 129^2 rows, 4.73 now)
 constexpr int MEMBER_W = 6;  // measured best of 6, 8 and 12 (rows of width 5 to 9 on the 2D hierarchies)
 
 template <class VA, class F>
@@ -87,22 +88,22 @@ __device__ __forceinline__ double member_row(const SellDesc &d, const MemberMat<
   const int32_t w = d.width;
   if (w <= 0) return 0.0;
   const int64_t v0 = d.vbase + lane, i0 = (int64_t)d.ibase + lane;
-  int32_t c[MEMBER_W];
-  VA a[MEMBER_W];
-#pragma unroll
-  for (int j = 0; j < MEMBER_W; j++) {
-    const int32_t jj = j < w ? j : w - 1;
-    c[j] = M.idx[i0 + (int64_t)64 * jj];
-    a[j] = M.val[v0 + (int64_t)64 * jj];
-  }
   double acc = 0.0;
+  for (int32_t j0 = 0; j0 < w; j0 += MEMBER_W) {
+    int32_t c[MEMBER_W];
+    VA a[MEMBER_W];
 #pragma unroll
-  for (int j = 0; j < MEMBER_W; j++) {
-    const double gv = f((int64_t)d.coff + c[j]);
-    acc += j < w ? (double)a[j] * gv : 0.0;
+    for (int j = 0; j < MEMBER_W; j++) {
+      const int32_t jj = j0 + j < w ? j0 + j : w - 1;
+      c[j] = M.idx[i0 + (int64_t)64 * jj];
+      a[j] = M.val[v0 + (int64_t)64 * jj];
+    }
+#pragma unroll
+    for (int j = 0; j < MEMBER_W; j++) {
+      const double gv = f((int64_t)d.coff + c[j]);
+      acc += j0 + j < w ? (double)a[j] * gv : 0.0;
+    }
   }
-  for (int32_t j = MEMBER_W; j < w; j++)
-    acc += (double)M.val[v0 + (int64_t)64 * j] * f((int64_t)d.coff + M.idx[i0 + (int64_t)64 * j]);
   return acc;
 }
 
@@ -187,6 +188,7 @@ __device__ void amg_member_vcycle(const MemberLevel<V> *__restrict__ T, int nt, 
       const VFVM_GLOBAL V *M = gmem(L.dinvA + L.doff[k]);
       for (int i = threadIdx.x; i < n; i += BS) {
         double acc = 0.0;
+#pragma unroll 8
         for (int c = 0; c < n; c++) acc += (double)M[(int64_t)i * n + c] * (double)b[r0 + c];
         out[r0 + i] = (V)acc;
       }
