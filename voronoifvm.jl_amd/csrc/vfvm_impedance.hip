@@ -11,8 +11,9 @@
 // frequency is a member of the batch, every kernel covers all members, converged
 // members drop out.  Scalar systems of some size are right-preconditioned by a multigrid
 // cycle that all frequencies of a group share (sweep_multigrid); the others, and what that
-// does not finish, run on the row scaling alone (sweep_jacobi).  Dot products are reduced in a fixed order (block partials, one
-// finishing block per member), so a sweep is deterministic.
+// does not finish, run on the row scaling alone (sweep_jacobi).  Dot products are reduced in
+// a fixed order (block partials, one finishing block per member), so a sweep is
+// deterministic.
 #include <algorithm>
 #include <cmath>
 #include <memory>
