@@ -10,11 +10,11 @@
 // Conventions: the operator is the row-scaled Jacobian  Ahat = S A  with
 // S = diag(1 / A_ii), which turns the 1e30 Dirichlet-penalty rows into unit
 // rows before any FP32 cast (1e30^2 would overflow an FP32 dot product).
-// Reductions: every reducing kernel writes one partial per block; a one-block
-// finalize kernel sums the partials in fixed order and runs a small "stage"
-// that updates the solver scalars in device memory (no cross-block fences,
-// deterministic sums).  Kernels of a finished solve return at entry, so the
-// host can enqueue several iterations between status reads.
+// Reductions: every reducing kernel writes one partial per block; the next kernel of the
+// solver (vfvm_bicgstab.h, vfvm_gmres.h) or a one-block finalize kernel sums the partials
+// in fixed order and runs a small "stage" that updates the solver scalars in device memory
+// (no cross-block fences, deterministic sums).  Kernels of a finished solve return at
+// entry, so the host can enqueue several iterations between status reads.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -301,27 +301,6 @@ __global__ void __launch_bounds__(VB) k_scale_rows(int64_t nnodes, const int32_t
       for (int i = 0; i < NS; i++)
 #pragma unroll
         for (int j = 0; j < NS; j++) binv[K * NS * NS + i * NS + j] = I[i][j];
-    }
-  }
-}
-
-// z = Binv r per node block (block-Jacobi on Ahat)
-template <int NS, class V>
-__global__ void __launch_bounds__(VB) k_blockjacobi(int64_t nnodes, const double *__restrict__ binv,
-                                                    const V *__restrict__ r, V *__restrict__ z, const KState *st,
-                                                    int skip_if_half) {
-  if (st && idle(st)) return;
-  if (st && skip_if_half && st->half) return;
-  for (int64_t K = (int64_t)blockIdx.x * VB + threadIdx.x; K < nnodes; K += (int64_t)gridDim.x * VB) {
-    double rv[NS];
-#pragma unroll
-    for (int j = 0; j < NS; j++) rv[j] = (double)r[K * NS + j];
-#pragma unroll
-    for (int i = 0; i < NS; i++) {
-      double acc = 0.0;
-#pragma unroll
-      for (int j = 0; j < NS; j++) acc += binv[K * NS * NS + i * NS + j] * rv[j];
-      z[K * NS + i] = (V)acc;
     }
   }
 }
@@ -707,15 +686,7 @@ void LinearSolver::prepare(const double *J, const vfvm_control_t &c, bool refact
 
 template <class V>
 const V *LinearSolver::precond(const V *r, V *z, KState *stp, int skip_if_half, const vfvm_control_t &c) {
-  const int ns = L.nspec;
-  if (c.precon == VFVM_PRECON_BLOCKJACOBI && ns > 1) {
-    unsigned g = grid_for(L.nnodes);
-    if (ns == 2)
-      hipLaunchKernelGGL((k_blockjacobi<2, V>), dim3(g), dim3(VB), 0, stream, L.nnodes, binv.p, r, z, stp, skip_if_half);
-    else
-      hipLaunchKernelGGL((k_blockjacobi<3, V>), dim3(g), dim3(VB), 0, stream, L.nnodes, binv.p, r, z, stp, skip_if_half);
-    return z;
-  } else if (c.precon == VFVM_PRECON_ILU0 || c.precon == VFVM_PRECON_ILU0_NATURAL) {
+  if (c.precon == VFVM_PRECON_ILU0 || c.precon == VFVM_PRECON_ILU0_NATURAL) {
     const IluStruct &I = *L.ilu;
     const V *lu = nullptr;
     if constexpr (sizeof(V) == 4) lu = ilu32s.p;
@@ -744,7 +715,8 @@ const V *LinearSolver::precond(const V *r, V *z, KState *stp, int skip_if_half, 
     amg.apply<V>(r, z, stp, skip_if_half, stream, L.probe);
     return z;
   }
-  // point Jacobi on the row-scaled operator is the identity
+  // point Jacobi on the row-scaled operator is the identity; node solves are part of the
+  // kernels that use them
   return r;
 }
 
